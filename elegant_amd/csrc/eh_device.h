@@ -129,6 +129,10 @@ typedef struct {
   int32_t csb_dense;        /* EO1 of the dense blocks at csb_dx0/csb_dy0 (5 or 6), else 0 */
   int32_t csb_dx0, csb_dy0;
   uint32_t csb_live;        /* dense blocks: bit t set if the t-th term (i-outer, j-inner) is non-zero */
+  /* how the regular path runs this element (eh_regular.h): 0 not at all; bends
+   * 1 without field terms, 2 with those of a gradient alone, 3 with any dense
+   * block; kick multipoles the order of their one term */
+  int32_t regular, reg_pad_;
 
   /* ---- RFCA ---- */
   int32_t rf_matrix, rf_nkicks, rf_same, rf_standing, rf_end1, rf_end2, rf_zero_volt;
@@ -604,6 +608,9 @@ EH_HD void eh_mface2(eh_p6 &p, const eh_desc &d, bool s_too) {
   }
 }
 
+EH_HD bool eh_mult_regular_n(const eh_desc &d, int pi, double &x, double &xp, double &y, double &yp, double &s,
+                             double dp);
+
 /* KQUAD/KSEXT/KOCT/KQUSE: multipole_tracking2 (src/multipole.c:660-1084) for one
  * particle, including the misalignment passes around the particle loop (method 0,
  * src/malign_mat.c:257-267, :580-590, tilt_matrices.c:156-187) and the loss
@@ -628,7 +635,14 @@ EH_HD int eh_multipole_t(eh_p6 &p, const eh_desc &d, int pi, const double *__res
   double dzLoss = 0;
   bool lost = false, entry = false;
   int how = 0; /* 0: coord untouched, 1: x,y written, 2: all written */
-  if (eh_isnan(x) || eh_isnan(xp) || eh_isnan(y) || eh_isnan(yp) || eh_fabs(x) > 10.0 || eh_fabs(y) > 10.0 ||
+  bool regular = false;
+  if constexpr (!RAD) {
+    if (d.regular)
+      regular = eh_mult_regular_n(d, pi, x, xp, y, yp, s, dp);
+  }
+  if (regular) {
+    how = 2;
+  } else if (eh_isnan(x) || eh_isnan(xp) || eh_isnan(y) || eh_isnan(yp) || eh_fabs(x) > 10.0 || eh_fabs(y) > 10.0 ||
       eh_fabs(xp) > 1.0 || eh_fabs(yp) > 1.0) {
     lost = entry = true;
   } else {
@@ -1316,6 +1330,8 @@ EH_HD void eh_edge_hwang(double &x, double &xp, double &y, double &yp, double dp
   yp = qy * f;
 }
 
+#include "eh_regular.h"
+
 /* CSBEND: track_through_csbend (src/csbend.c:1088-1403) for one particle, with
  * integrate_csbend_ordn (src/csbend.c:1459-1720) and the canonical conversions
  * (:1436-1454).  Returns true if lost.  RAD and FULL as for eh_multipole_t. */
@@ -1376,8 +1392,12 @@ EH_HD bool eh_csbend_t(eh_p6 &p, const eh_desc &d, int pi, const eh_fterm *__res
   double rh = 0, rl = 0;
   const bool rok = !RAD && eh_recip_pair(b1, rh, rl);
   double dist = 0, dz_lost = 0;
-  bool lost = false;
-  for (int i = 0; i < d.csb_nslices && !lost; i++) {
+  bool lost = false, regular = false;
+  if constexpr (!RAD) {
+    if (d.regular)
+      regular = eh_csb_regular_n(d, pi, terms, b1, rh, X, QX, Y, QY, dist);
+  }
+  for (int i = 0; i < d.csb_nslices && !lost && !regular; i++) {
     if (!eh_ap_ok<FULL>(X, Y, apx, apy, d.ap_rtilt, d.ap_cs0, d.ap_cs1, ell, d.ell_xe[pi], d.ell_ye[pi])) {
       lost = true;
       break;
@@ -1446,7 +1466,7 @@ EH_HD bool eh_csbend_t(eh_p6 &p, const eh_desc &d, int pi, const eh_fterm *__res
   }
   if (!lost) {
     dz_lost = d.csb_dzl;
-    if (!eh_ap_ok<FULL>(X, Y, apx, apy, d.ap_rtilt, d.ap_cs0, d.ap_cs1, ell, d.ell_xe[pi], d.ell_ye[pi]))
+    if (!regular && !eh_ap_ok<FULL>(X, Y, apx, apy, d.ap_rtilt, d.ap_cs0, d.ap_cs1, ell, d.ell_xe[pi], d.ell_ye[pi]))
       lost = true;
     else
       S4 += dist;

@@ -347,6 +347,11 @@ static long build_multipole(eh_desc *d, const EH_ELEMENT_LIST *e, const eh_ctx &
   d->ap_cs0 = eh_cos(rt);
   d->ap_cs1 = eh_sin(rt);
   d->length = drift;
+  /* the regular path: one term, an untilted rectangular aperture, a length (the
+   * radiation block's round trip runs) and the exact Hamiltonian */
+  if (!expand && mdrift != 0 && !d->ap_rtilt && !d->ell_any && d->mp_order[0] && !d->mp_order[1] && !d->mp_order[2] &&
+      !skew[0])
+    d->regular = d->mp_order[0];
   return EH_OK;
 }
 
@@ -383,6 +388,23 @@ static void csbend_coefficients(const EH_CSBEND *cb, double b[9], double cc[9]) 
   cc[2] *= (1 + cb->fse) / (1 + cb->fse + cb->fseDipole);
   b[0] = cb->xKick / cb->angle;
   cc[0] = cb->yKick / cb->angle;
+}
+
+/* which regular path a bend takes (eh_regular.h): it needs divisions by the radii
+ * through their reciprocals, positive radii (a zero quotient keeps its sign), an
+ * untilted rectangular aperture and sub-step angles below 2^-4, where the shared
+ * sin and cos are their short series */
+static int32_t csb_regular(const eh_desc &d) {
+  if (!d.csb_recip || !(d.rho0 > 0) || !(d.rho_actual > 0) || d.ap_rtilt || d.ell_any)
+    return 0;
+  for (int j = 0; j < d.nsub; j++)
+    if (!(std::fabs(d.csb_dshr[j]) < 0x1p-4))
+      return 0;
+  if (!d.csb_field)
+    return 1;
+  if (d.csb_dense == 5 && d.csb_live == EH_LIVE_GRADIENT)
+    return 2;
+  return d.csb_dense ? 3 : 0;
 }
 
 static long build_csbend(eh_desc *d, const EH_CSBEND *cb, const eh_ctx &c, std::vector<eh_fterm> &pool) {
@@ -554,6 +576,7 @@ static long build_csbend(eh_desc *d, const EH_CSBEND *cb, const eh_ctx &c, std::
     d->csb_ds[j] = s * kickFrac[j];
   }
   d->csb_dzl = cb->nSlices * s;
+  d->regular = csb_regular(*d);
   d->csb_edge1 = (cb->edgeFlags & EH_BEND_EDGE1_EFFECTS) && cb->edge1_effects >= 1;
   d->csb_edge2 = (cb->edgeFlags & EH_BEND_EDGE2_EFFECTS) && cb->edge2_effects >= 1;
   d->csb_esimple1 = d->csb_edge1 && cb->edge1_effects == 3;

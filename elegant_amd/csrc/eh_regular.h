@@ -1,0 +1,362 @@
+/* eh_regular.h -- the integrators for regular particles.
+ *
+ * Nearly every particle of every beam is regular: inside the apertures, with
+ * slopes of milliradians and a momentum within some percent of the reference.
+ * For those the general maps spend most of their instructions on what cannot
+ * happen: the range scaling and special cases of IEEE division and square root,
+ * the branches of the transcendental functions, the loss bookkeeping.  The
+ * integrators here leave all of that out, keep one flag per particle that says
+ * it stayed regular, and are thrown away for a particle that did not: the caller
+ * runs the general integrator for it from the saved entry state.
+ *
+ * Every result is the general integrator's, bit for bit.  Sums, products and
+ * polynomials are the same operations in the same order.  Quotients and roots
+ * are correctly rounded here too, by other means:
+ *
+ *  - RN(a / b) from y = RN(1 / b): q = RN(a y) is within 1.5 ulp, its residual
+ *    is exact in one fma, and RN(q + residual y) is the correctly rounded
+ *    quotient (P. Markstein, IBM J. Res. Develop. 34 (1990) 111-119), for normal
+ *    quotients away from underflow.  The residual is formed with its sign
+ *    reversed, which keeps the sign of a zero numerator over a positive b.
+ *  - y = RN(1 / b) from y0 within a few ulps: one Newton step y0 + y0 e with
+ *    e = 1 - b y0 exact is 1 / b to 2^-101 before its only rounding.  That decides
+ *    the rounding unless b = 2^n (1 - k 2^-53) with a small odd k, where 1 / b lies
+ *    only k^2 2^-106 above a midpoint; there y must come out above it (the
+ *    quotient of a power of two by 1 - 2^-53 is wrong otherwise), which the two
+ *    routines below arrange each in its way.  Elsewhere a y off by 2^-27 of a half
+ *    ulp more still gives the correctly rounded quotient, since b^2 is then below
+ *    4 by more than that.
+ *  - RN(sqrt a) from g within a few ulps: g + (a - g g) h with a - g g exact and
+ *    h = 1 / (2 g) to 2^-50 is sqrt a to 2^-101 before its only rounding.
+ *
+ * What bounds these loops is the number of instructions: a dependent FP64 fma
+ * issues every 5 cycles from one wavefront and every 4 from several, so that a
+ * launch of few particles gains nothing from independent operations and one of
+ * many nothing from latency hiding.  A sub-step of a gradient bend takes 165
+ * vector and 30 scalar instructions here against 270 and 215 in the general
+ * integrator, whose branches also keep the compiler from holding the polynomial
+ * constants in scalar registers.  Measured (MI355X, MBA ring, fused, 2 turns): 1e6
+ * particles 283 -> 166 ms, 30 401 particles (one wavefront on half of the SIMDs)
+ * 48.4 -> 21.4 ms; FODO ring, 1e4 particles, 40 turns 27.2 -> 13.4 ms.  A
+ * wavefront with one irregular particle pays for both integrators of that
+ * element; on a grid filling the aperture of the MBA ring no particle that is not
+ * lost ever leaves the limits below.
+ *
+ * The starting values need no hardware estimate (v_rcp_f64 and v_rsq_f64 give 24
+ * bits and take the issue time of four fma): a bend's and a multipole's root is
+ * of (1 + delta)^2 minus a small square, so the binomial series around
+ * 1 / (1 + delta), formed once per element, is accurate to the last bits, and a
+ * cosine close to one is its own estimate.  Only IEEE +, -, *, and fma are used,
+ * so that the host build of these routines gives the same doubles.
+ */
+#ifndef EH_REGULAR_H
+#define EH_REGULAR_H
+
+/* limits of the regular path: 1 + delta, canonical momenta (about the slopes; a
+ * bend's QX swings by its sub-step angles on the design orbit already), and the
+ * smallest non-zero momentum, whose quotients are far from underflow.  With them
+ * the series argument below is < 2^-11 and |sin phi| < 2^-4. */
+#define EH_REG_B1_MIN 0.875
+#define EH_REG_B1_MAX 1.25
+#define EH_REG_QMAX 0.0117
+#define EH_REG_QXMAX 0.05
+#define EH_REG_QMIN 0x1p-340
+/* dense 5 x 5 field block: the terms a gradient alone leaves, (i, j) = (0, 0..4),
+ * (1, 0), (1, 2), (1, 3), (2, 2) */
+#define EH_LIVE_GRADIENT 0x9bfu
+
+/* RN(a / b) with y = RN(1 / b), b > 0 */
+EH_HD double eh_reg_div(double a, double b, double y) {
+  const double q = a * y;
+  return eh_fma(-eh_fma(q, b, -a), y, q);
+}
+
+/* f = RN(sqrt a) and y = RN(1 / f) for a = b1^2 (1 - w) up to its rounding, from
+ * rh = RN(1 / b1) and w < 2^-11: the binomial series of (1 - w)^-1/2 to w^4 (the
+ * next term is below 2^-56) */
+EH_HD void eh_reg_root(double a, double w, double rh, double &f, double &y) {
+  double t = eh_fma(w, 0x1.18p-2, 0x1.4p-2);
+  t = eh_fma(w, t, 0x1.8p-2);
+  t = eh_fma(w, t, 0.5);
+  const double y0 = eh_fma(rh * w, t, rh);
+  const double g = a * y0;
+  f = eh_fma(eh_fma(-g, g, a), 0.5 * y0, g);
+  /* 2^-80: far below the last bit, far above the 2^-101 by which the step falls
+   * short, so that 1 / f just above a midpoint (see the top) rounds up */
+  y = eh_fma(eh_fma(-f, y0, 1.0) + 0x1p-80, y0, y0);
+}
+
+/* RN(1 / c) for a cosine c = 1 - u, 0 <= u < 2^-9: 2 - c is 1 / c to u^2; one
+ * step of third order leaves 3 quarters of an ulp, one of second order the
+ * correct rounding.  Starting 2^-51 too high makes 1 - 2^-53 come out right: both
+ * steps then end above the midpoint, at 1 + 2^-52. */
+EH_HD double eh_reg_recip1(double c) {
+  const double y0 = 0x1.0000000000001p1 - c;
+  const double e = eh_fma(-c, y0, 1.0);
+  const double y1 = eh_fma(y0, eh_fma(e, e, e), y0);
+  return eh_fma(eh_fma(-c, y1, 1.0), y1, y1);
+}
+
+/* eh_asin below 2^-4: the two short series of eh_asin_small */
+EH_HD double eh_reg_asin(double x) {
+  const double z = x * x;
+  double q = EH_ASIN_4;
+  const bool longer = !(eh_fabs(x) < 0x1p-8);
+#if defined(__HIP_DEVICE_COMPILE__)
+  if (__ballot(longer))
+#else
+  if (longer)
+#endif
+  {
+    double p = EH_ASIN_7;
+    p = EH_ASIN_6 + z * p;
+    p = EH_ASIN_5 + z * p;
+    p = EH_ASIN_4 + z * p;
+    q = longer ? p : q;
+  }
+  q = EH_ASIN_3 + z * q;
+  q = EH_ASIN_2 + z * q;
+  q = EH_ASIN_1 + z * q;
+  return eh_fma(x * z, q, x);
+}
+
+/* the field of a bend that has a gradient and nothing else, from the nine terms
+ * of its dense block in the order of eh_csb_fields_dense; 0 + c y is one fma */
+struct eh_grad_field {
+  double y1, y2c, y3, y4, x1, x1y2, x1y3, x2y2, c0;
+};
+
+EH_HD eh_grad_field eh_grad_load(const eh_fterm *__restrict__ cx, const eh_fterm *__restrict__ cy) {
+  return {cx[1].coef, cy[2].coef, cx[3].coef, cy[4].coef, cy[5].coef, cy[7].coef, cx[8].coef, cy[12].coef, cy[0].coef};
+}
+
+EH_HD void eh_grad_eval(const eh_grad_field &c, double x, double y, double &Fx, double &Fy) {
+  const double y2 = y * y, y3 = y2 * y, y4 = y3 * y;
+  Fx = eh_fma(c.y1, y, 0.0);
+  Fy = c.c0 + c.y2c * y2;
+  Fx += c.y3 * y3;
+  Fy += c.y4 * y4;
+  Fy += c.x1 * x;
+  Fy += c.x1y2 * x * y2;
+  Fx += c.x1y3 * x * y3;
+  Fy += c.x2y2 * (x * x) * y2;
+}
+
+/* slopes of regular momenta (convertMomentaToSlopes) */
+struct eh_reg_slopes {
+  double xp, yp, f, y;
+};
+
+EH_HD eh_reg_slopes eh_reg_m2s(double qx, double qy, double b1s, double rh, double rh2) {
+  eh_reg_slopes s;
+  const double x2 = qx * qx, y2 = qy * qy;
+  eh_reg_root(b1s - x2 - y2, (x2 + y2) * rh2, rh, s.f, s.y);
+  s.xp = eh_reg_div(qx, s.f, s.y);
+  s.yp = eh_reg_div(qy, s.f, s.y);
+  return s;
+}
+
+/* zero, or far above underflow */
+EH_HD bool eh_reg_sized(double ax) { return ax >= EH_REG_QMIN || ax == 0; }
+
+/* the field sums of one kick of order N, eh_mkick's terms and order (0 + v is
+ * v + 0, one fma where v is a product) */
+template <int ORDER> EH_HD void eh_reg_mfield(double x, double y, double &Fx, double &Fy) {
+  if constexpr (ORDER == 1) {
+    Fy = 0.0 + x;
+    Fx = 0.0 + y;
+  } else if constexpr (ORDER == 2) {
+    Fy = eh_fma(0.5, x * x, 0.0);
+    Fx = eh_fma(x, y, 0.0);
+    Fy += -0.5 * (y * y);
+  } else {
+    const double x2 = x * x, y2 = y * y;
+    Fy = eh_fma(1. / 6., x2 * x, 0.0);
+    Fx = eh_fma(0.5 * x2, y, 0.0);
+    Fy += -0.5 * x * y2;
+    Fx += -(1. / 6.) * (y2 * y);
+  }
+}
+
+/* integrate_kick_multipole_ordn without losses for a regular particle and one
+ * term of the given order: slopes to momenta, the slices, and back; x, xp, y,
+ * yp, s advance through the element if it returns true and are left alone
+ * otherwise.  (1 + x'^2 + y'^2)^1/2 of a sub-step is (1 + delta) / f up to
+ * roundings, which one correction step removes.  The exit's slopes are those of
+ * the last kick. */
+template <int ORDER>
+EH_HD bool eh_mult_regular(const eh_desc &d, int pi, double &x_, double &xp_, double &y_, double &yp_, double &s_,
+                           double dp) {
+  double x = x_, y = y_, s = 0;
+  const double mdx = d.mdx, mdy = d.mdy;
+  const double apx = d.ap_xmax[pi] > 0 ? d.ap_xmax[pi] : 0x1p60, apy = d.ap_ymax[pi] > 0 ? d.ap_ymax[pi] : 0x1p60;
+  const double b1 = 1 + dp;
+  bool bad = !(b1 >= EH_REG_B1_MIN && b1 <= EH_REG_B1_MAX && eh_fabs(x) <= 10.0 && eh_fabs(y) <= 10.0 &&
+               eh_fabs(xp_) <= EH_REG_QMAX && eh_fabs(yp_) <= EH_REG_QMAX && eh_reg_sized(eh_fabs(xp_)) &&
+               eh_reg_sized(eh_fabs(yp_)));
+#if defined(__HIP_DEVICE_COMPILE__)
+  if (__ballot(!bad) == 0)
+    return false;
+#else
+  if (bad)
+    return false;
+#endif
+  const double b1s = b1 * b1, rh = 1.0 / b1, rh2 = rh * rh, hrh = 0.5 * rh;
+  double qx, qy;
+  {
+    const double u = eh_sqr(xp_) + eh_sqr(yp_);
+    double w, yw;
+    eh_reg_root(1 + eh_sqr(xp_) + eh_sqr(yp_), -u, 1.0, w, yw);
+    qx = eh_reg_div(b1 * xp_, w, yw);
+    qy = eh_reg_div(b1 * yp_, w, yw);
+  }
+  eh_reg_slopes v = eh_reg_m2s(qx, qy, b1s, rh, rh2);
+  const int nsl = d.nslices, nsub = d.nsub;
+  for (int ik = 0; ik < nsl; ik++) {
+    bad = bad || !(eh_fabs(x + mdx) <= apx && eh_fabs(y + mdy) <= apy);
+    for (int step = 0; step < nsub; step++) {
+      const double dsh = d.dsh[step];
+      x += v.xp * dsh;
+      y += v.yp * dsh;
+      const double a2 = 1 + eh_sqr(v.xp) + eh_sqr(v.yp);
+      const double g = b1 * v.y;
+      s += dsh * eh_fma(eh_fma(-g, g, a2), hrh * v.f, g);
+      if (step == nsub - 1)
+        break;
+      double Fx, Fy;
+      eh_reg_mfield<ORDER>(x, y, Fx, Fy);
+      const double K = d.kick[step][0];
+      qx -= K * Fy;
+      qy += K * Fx;
+      if (d.has_xkick) { /* eh_mkick<0>: the other plane gains a signed zero */
+        qx -= d.xk[step];
+        qy += d.xk[step] * 0.0;
+      }
+      if (d.has_ykick) {
+        qx -= d.yk[step] * 0.0;
+        qy -= d.yk[step];
+      }
+      const double ax = eh_fabs(qx), ay = eh_fabs(qy);
+      bad = bad || !(ax <= EH_REG_QMAX && ay <= EH_REG_QMAX);
+      if (!(ax >= EH_REG_QMIN && ay >= EH_REG_QMIN))
+        bad = bad || !(eh_reg_sized(ax) && eh_reg_sized(ay));
+      /* the radiation block's division and multiplication by 1 + delta */
+      qx = eh_reg_div(qx, b1, rh) * b1;
+      qy = eh_reg_div(qy, b1, rh) * b1;
+      v = eh_reg_m2s(qx, qy, b1s, rh, rh2);
+    }
+  }
+  bad = bad || !(eh_fabs(x + mdx) <= apx && eh_fabs(y + mdy) <= apy && eh_fabs(x) <= 10.0 && eh_fabs(y) <= 10.0);
+  if (bad)
+    return false;
+  x_ = x;
+  xp_ = v.xp;
+  y_ = y;
+  yp_ = v.yp;
+  s_ = s;
+  return true;
+}
+
+EH_HD bool eh_mult_regular_n(const eh_desc &d, int pi, double &x, double &xp, double &y, double &yp, double &s,
+                             double dp) {
+  if (d.regular == 1)
+    return eh_mult_regular<1>(d, pi, x, xp, y, yp, s, dp);
+  if (d.regular == 2)
+    return eh_mult_regular<2>(d, pi, x, xp, y, yp, s, dp);
+  return eh_mult_regular<3>(d, pi, x, xp, y, yp, s, dp);
+}
+
+/* integrate_csbend_ordn without losses for a regular particle: X, QX, Y, QY and
+ * the path `dist` advance through the bend if it returns true and are left alone
+ * otherwise.  FIELD as eh_desc.regular. */
+template <int FIELD>
+EH_HD bool eh_csb_regular(const eh_desc &d, int pi, const eh_fterm *__restrict__ terms, double b1, double rh,
+                          double &X_, double &QX_, double &Y_, double &QY_, double &dist_) {
+  double X = X_, QX = QX_, Y = Y_, QY = QY_, dist = 0;
+  const double rho0 = d.rho0, rho_a = d.rho_actual, r0h = d.rho0_rh, rah = d.rhoa_rh;
+  const double apx = d.ap_xmax[pi] > 0 ? d.ap_xmax[pi] : 0x1p60, apy = d.ap_ymax[pi] > 0 ? d.ap_ymax[pi] : 0x1p60;
+  const double b1s = b1 * b1, rh2 = rh * rh;
+  eh_grad_field gf;
+  if constexpr (FIELD == 2)
+    gf = eh_grad_load(terms + d.csb_dx0, terms + d.csb_dy0);
+  bool bad = !(b1 >= EH_REG_B1_MIN && b1 <= EH_REG_B1_MAX && eh_fabs(QY) <= EH_REG_QMAX &&
+               (eh_fabs(QY) >= EH_REG_QMIN || QY == 0));
+  /* f and 1 / f depend on QY alone, which drifts leave unchanged: formed at
+   * entry and after every kick */
+  double f, y;
+  {
+    const double q2 = QY * QY;
+    eh_reg_root(b1s - q2, q2 * rh2, rh, f, y);
+  }
+  const int nsl = d.csb_nslices, nsub = d.nsub;
+  for (int i = 0; i < nsl; i++) {
+    bad = bad || !(eh_fabs(X) <= apx && eh_fabs(Y) <= apy && eh_fabs(QX) <= EH_REG_QXMAX &&
+                   eh_fabs(QX) >= EH_REG_QMIN);
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (__ballot(!bad) == 0)
+      break;
+#else
+    if (bad)
+      break;
+#endif
+    for (int j = 0; j < nsub; j++) {
+      const double sin_phi = eh_reg_div(QX, f, y);
+      const double phi = eh_reg_asin(sin_phi);
+      const double ang = d.csb_dshr[j] + phi;
+      bad = bad || !(eh_fabs(ang) < 0x1p-4); /* the short series of eh_sincos */
+      const double sine = eh_sin_poly(ang), cosi = eh_cos_poly(ang);
+      const double yc = eh_reg_recip1(cosi);
+      const double tang = eh_reg_div(sine, cosi, yc);
+      const double cos_phi = eh_cos_poly(phi);
+      QX = f * sine;
+      const double tphi = eh_reg_div(sin_phi, cos_phi, eh_reg_recip1(cos_phi));
+      const double factor = eh_reg_div((rho0 + X) * cos_phi, f, y) * (tang - tphi);
+      Y += QY * factor;
+      dist += factor * b1;
+      const double fr = eh_reg_div(cos_phi, cosi, yc);
+      X = rho0 * (fr - 1) + fr * X;
+      if (j == nsub - 1)
+        break;
+      const double u = d.csb_ds[j] * (1 + eh_reg_div(X, rho0, r0h));
+      double Fx = 0, Fy = 1;
+      if constexpr (FIELD == 2)
+        eh_grad_eval(gf, X, Y, Fx, Fy);
+      if constexpr (FIELD == 3)
+        eh_csb_fields(d, terms, X, Y, Fx, Fy);
+      const double ny = u * Fx;
+      QX -= eh_reg_div(u * Fy, rho_a, rah);
+      QY += eh_reg_div(ny, rho_a, rah);
+      /* a momentum far above underflow has lost nothing to an inexact tiny
+       * kick; a particle in the mid-plane keeps QY = 0 exactly */
+      const double ax = eh_fabs(QX), ay = eh_fabs(QY);
+      bad = bad || !(ax <= EH_REG_QXMAX && ay <= EH_REG_QMAX);
+      if (!(ax >= EH_REG_QMIN && ay >= EH_REG_QMIN))
+        bad = bad || !(ax >= EH_REG_QMIN && QY == 0 && ny == 0);
+      /* the radiation block's division and multiplication by 1 + delta */
+      QX = eh_reg_div(QX, b1, rh) * b1;
+      QY = eh_reg_div(QY, b1, rh) * b1;
+      const double q2 = QY * QY;
+      eh_reg_root(b1s - q2, q2 * rh2, rh, f, y);
+    }
+  }
+  bad = bad || !(eh_fabs(X) <= apx && eh_fabs(Y) <= apy);
+  if (bad)
+    return false;
+  X_ = X;
+  QX_ = QX;
+  Y_ = Y;
+  QY_ = QY;
+  dist_ = dist;
+  return true;
+}
+
+EH_HD bool eh_csb_regular_n(const eh_desc &d, int pi, const eh_fterm *__restrict__ terms, double b1, double rh,
+                            double &X, double &QX, double &Y, double &QY, double &dist) {
+  if (d.regular == 2)
+    return eh_csb_regular<2>(d, pi, terms, b1, rh, X, QX, Y, QY, dist);
+  if (d.regular == 1)
+    return eh_csb_regular<1>(d, pi, terms, b1, rh, X, QX, Y, QY, dist);
+  return eh_csb_regular<3>(d, pi, terms, b1, rh, X, QX, Y, QY, dist);
+}
+
+#endif

@@ -322,3 +322,81 @@ extern "C" long bh_track(const double *flat, const long *counts, long nvar, EH_E
     return fail(EH_ERR_STATE, "bh_track: %ld alive + %ld lost != %ld", total, n_grave, idn);
   return total;
 }
+
+/* the quotients and roots of the regular path (eh_regular.h) against IEEE
+ * division and square root: roots of b1^2 (1 - w) and quotients by them, by
+ * cosines and by 1 + delta, half of the numerators next to a rounding midpoint,
+ * divisors a few units in the last place below one among them.  Returns the
+ * number of results that differ in any bit. */
+extern "C" long bh_regular_arithmetic(long n, unsigned seed) {
+  std::mt19937_64 rng(seed);
+  auto uni = [&](double lo, double hi) { return lo + (hi - lo) * (double)(rng() >> 11) * 0x1p-53; };
+  long bad = 0;
+  for (long k = 0; k < n; k++) {
+    double b1 = (k & 3) == 0 ? 1.0 + std::ldexp((double)(int)(rng() % 17) - 8, -53) : uni(EH_REG_B1_MIN, EH_REG_B1_MAX);
+    if ((k & 3) == 1)
+      b1 = 1.0;
+    const double rh = 1.0 / b1;
+    /* squares from underflow to the limit */
+    const double q = std::ldexp(uni(0.5, 1), -(int)(rng() % ((k & 4) ? 40 : 400))) * EH_REG_QMAX;
+    const double p = (k & 8) ? 0.0 : std::ldexp(uni(0.5, 1), -(int)(rng() % 40)) * EH_REG_QMAX;
+    const double a = (b1 * b1 - p * p) - q * q;
+    double f, y;
+    eh_reg_root(a, (p * p + q * q) * (rh * rh), rh, f, y);
+    bad += eh_bits(f) != eh_bits(std::sqrt(a));
+    const double c = eh_cos_poly(std::ldexp(uni(0.5, 1), -(int)(rng() % 30)) * 0x1p-4);
+    const double div[3] = {f, c, b1}, rec[3] = {y, eh_reg_recip1(c), rh};
+    for (int m = 0; m < 3; m++) {
+      const double b = div[m];
+      double num = std::ldexp(uni(0.5, 1), -(int)(rng() % 300));
+      if (k & 16) {
+        const double t = uni(0.5, 2), mid = t + std::ldexp((rng() & 1) ? 1.0 : -1.0, std::ilogb(t) - 53);
+        num = b * mid;
+        const int w = (int)(rng() % 3);
+        if (w)
+          num = std::nextafter(num, w == 1 ? INFINITY : -INFINITY);
+      } else if ((k & 0x3e0) == 0) {
+        num = std::ldexp(1.0, -(int)(rng() % 300)); /* a power of two */
+      }
+      if ((rng() & 63) == 0)
+        num = 0;
+      if (rng() & 1)
+        num = -num;
+      bad += eh_bits(eh_reg_div(num, b, rec[m])) != eh_bits(num / b);
+    }
+  }
+  return bad;
+}
+
+/* how many of n particles (rows of 6 coordinates) the regular path takes
+ * through one kick multipole or bend (0 if the element has no regular path);
+ * taken[i] tells which */
+extern "C" long bh_regular_taken(const double *z, long n, const EH_ELEMENT_LIST *e, double xmax, double ymax, double Po,
+                                 int32_t *taken) {
+  EH_MAXAMP amp = {};
+  amp.x_max = xmax;
+  amp.y_max = ymax;
+  eh_ctx c = {};
+  c.Po = Po;
+  c.ap[0] = c.ap[1] = &amp;
+  eh_desc d;
+  std::vector<eh_fterm> terms;
+  long r = build_desc(&d, e, c, terms);
+  if (r < 0)
+    return r;
+  long count = 0;
+  for (long i = 0; i < n; i++) {
+    double x = z[6 * i], xp = z[6 * i + 1], y = z[6 * i + 2], yp = z[6 * i + 3], s = 0;
+    const double b1 = 1 + z[6 * i + 5];
+    taken[i] = 0;
+    if (d.regular && d.type == EH_T_CSBEND) {
+      const double f = b1 / eh_sqrt(1 + xp * xp + yp * yp);
+      double QX = xp * f, QY = yp * f;
+      taken[i] = eh_csb_regular_n(d, 0, terms.data(), b1, 1.0 / b1, x, QX, y, QY, s);
+    } else if (d.regular) {
+      taken[i] = eh_mult_regular_n(d, 0, x, xp, y, yp, s, z[6 * i + 5]);
+    }
+    count += taken[i];
+  }
+  return count;
+}

@@ -1,0 +1,149 @@
+"""The integrators for regular particles against the oracle, where they can go
+wrong: at and beyond every limit at which a particle leaves them for the general
+ones, at zeros of either sign and near underflow.  Bit for bit, signs of zeros
+included; no tolerance."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from elegant_amd import configs, structs as S, tracking
+from elegant_amd.lattice import Element, Lattice
+from oracle import oracle
+from tests.test_batch_host import _host_track, harness
+
+Po = configs.p_central_from_mev(3000.0)
+BEND = dict(L=0.8, ANGLE=0.0314, N_KICKS=3, EDGE1_EFFECTS=0, EDGE2_EFFECTS=0)
+
+# element, and the regular path its descriptor asks for
+ELEMENTS = {
+    "bend": (Element("B", "CSBEND", **BEND), True),
+    "bend_edges": (Element("B", "CSBEND", **{**BEND, "EDGE1_EFFECTS": 1, "EDGE2_EFFECTS": 1, "E1": 0.01, "HGAP": 0.01}),
+                   True),
+    "bend_k1": (Element("B", "CSBEND", K1=-0.5, FSE=1e-3, **BEND), True),
+    "bend_k1_order2": (Element("B", "CSBEND", K1=0.5, INTEGRATION_ORDER=2, **BEND), True),
+    "bend_k1_order6": (Element("B", "CSBEND", K1=0.5, INTEGRATION_ORDER=6, **BEND), True),
+    "bend_k1_k2": (Element("B", "CSBEND", K1=0.5, K2=3.0, **BEND), True),
+    "bend_k3": (Element("B", "CSBEND", K3=30.0, **BEND), True),
+    "bend_wide_angle": (Element("B", "CSBEND", **{**BEND, "ANGLE": 0.15}), True),
+    "bend_steep_steps": (Element("B", "CSBEND", **{**BEND, "ANGLE": 0.5}), False),
+    "bend_negative": (Element("B", "CSBEND", K1=0.3, **{**BEND, "ANGLE": -0.0314}), False),
+    "bend_tilted": (Element("B", "CSBEND", K1=0.3, TILT=0.1, **BEND), False),
+    "quad": (Element("Q", "KQUAD", L=0.25, K1=2.9, N_KICKS=8), True),
+    "quad_offset_kicks": (Element("Q", "KQUAD", L=0.25, K1=-1.4, N_KICKS=8, DX=3e-5, DY=-2e-5, DZ=1e-5, FSE=1e-3,
+                                  HKICK=1e-5, VKICK=-2e-5), True),
+    "quad_order2": (Element("Q", "KQUAD", L=0.25, K1=1.0, N_KICKS=3, INTEGRATION_ORDER=2), True),
+    "quad_order6": (Element("Q", "KQUAD", L=0.25, K1=1.0, N_KICKS=12, INTEGRATION_ORDER=6), True),
+    "quad_tilted": (Element("Q", "KQUAD", L=0.25, K1=1.0, N_KICKS=8, TILT=0.2), False),
+    "quad_thin": (Element("Q", "KQUAD", L=0.0, K1=1.0, N_KICKS=8), False),
+    "quad_off": (Element("Q", "KQUAD", L=0.25, K1=0.0, N_KICKS=8), False),
+    "sext": (Element("X", "KSEXT", L=0.2, K2=-25.0, N_KICKS=4), True),
+    "sext_k1": (Element("X", "KSEXT", L=0.2, K2=-25.0, K1=0.1, N_KICKS=4), False),
+    "oct": (Element("O", "KOCT", L=0.2, K3=-1000.0), True),
+}
+APERTURE = 0.02
+
+
+def particles():
+    """ordinary particles, and one or a pair beyond the limits at a time"""
+    rng = np.random.default_rng(2)
+    z = [[3e-3 * u[0], 5e-4 * u[1], 2e-3 * u[2], 5e-4 * u[3], 1e-3 * u[4], 2e-3 * u[5]]
+         for u in rng.standard_normal((48, 6))]
+    base = [1.3e-3, 2.1e-4, -7e-4, 3.3e-4, 1e-3, 4e-4]
+    nxt = np.nextafter
+
+    def put(k, values):
+        for v in values:
+            p = list(base)
+            p[k] = v
+            z.append(p)
+
+    around = lambda v: [nxt(v, 0), v, nxt(v, 1e9)]  # noqa: E731
+    lim = around(APERTURE) + around(10.0)
+    put(0, lim + [-v for v in lim] + [0.0, -0.0, 1e-300, 5e-324, np.inf, np.nan])
+    put(2, lim + [0.0, -0.0, -1e-300, 5e-324, -np.inf, np.nan])
+    slope = around(2.0 ** -8) + around(0.0117) + around(0.05) + around(0.0625) + [0.0116, 0.0118, 0.3]
+    tiny = [0.0, -0.0, 1e-300, -1e-300, 2e-103, 4e-103, 5e-324, np.inf, np.nan]
+    put(1, slope + [-v for v in slope] + tiny)
+    put(3, slope + [-v for v in slope] + tiny)
+    put(5, around(-0.125) + around(0.25) + [-0.3, 0.5, -0.999, -1.0, -1.5, 0.0, 2.0 ** -53, -2.0 ** -53, np.nan])
+    for p in ([0.0] * 6, [-0.0] * 6, [1e-3, 0, 0, 0, 0, 0], [0, 0, 1e-3, 0, 0, 0], [1e-3, -0.0, -0.0, -0.0, 0, 0],
+              [1e-3, 1e-4, 1e-300, 0, 0, 0], [1e-3, 1e-4, 0, 1e-300, 0, 0], [1e-3, 1e-4, 1e-160, 1e-200, 0, 1e-3],
+              [2e-310, 1e-310, 3e-310, 1e-310, 0, 0]):
+        z.append(list(p))
+    rows = np.zeros((len(z), S.NPROP))
+    rows[:, :6] = z
+    rows[:, 6] = np.arange(1, len(z) + 1)
+    return rows
+
+
+def line(name):
+    return Lattice([Element("AP", "MAXAMP", X_MAX=APERTURE, Y_MAX=APERTURE), ELEMENTS[name][0]])
+
+
+def identical(got, ref):
+    """doubles equal, NaN for NaN, zeros of one sign"""
+    return ((got == ref) & (np.signbit(got) == np.signbit(ref))) | (np.isnan(got) & np.isnan(ref))
+
+
+def check(got, ref, what):
+    bad = np.argwhere(~identical(got, ref))
+    assert not len(bad), "%s: %d entries differ, first at id %d column %d: %r, oracle %r" % (
+        what, len(bad), ref[bad[0][0], 6] if ref.shape[1] > 6 else -1, bad[0][1], got[tuple(bad[0])],
+        ref[tuple(bad[0])])
+
+
+def test_quotients_and_roots_are_correctly_rounded():
+    assert harness().bh_regular_arithmetic(400000, 5) == 0
+
+
+@pytest.mark.parametrize("name", sorted(ELEMENTS))
+def test_host_build_matches_oracle(name):
+    rows = particles()
+    r, out6, lpass, _ = _host_track([rows], [line(name)], 2, Po, None, 1)
+    ref, n, _, _ = oracle.do_tracking(rows, line(name), 2, Po)
+    assert r == n
+    got = ref.copy()
+    where = ref[:, 6].astype(int) - 1
+    got[:, :6] = out6[where]
+    # the position of a loss at entry, or in an element with an exit offset, is settled on download
+    settled = (lpass[where] != -1) & ((lpass[where] & 0x40000000 != 0) | ("DZ" in ELEMENTS[name][0].params))
+    got[settled, 4] = ref[settled, 4]
+    check(got, ref, name)
+
+
+@pytest.mark.parametrize("name", sorted(ELEMENTS))
+def test_who_is_regular(name):
+    """ordinary particles take the regular path of every element that has one,
+    particles beyond a limit do not"""
+    el, has = ELEMENTS[name]
+    arr, keep = Lattice([el]).c_beamline()
+    rows = particles()
+    z = np.ascontiguousarray(rows[:, :6])
+    taken = np.zeros(len(z), dtype=np.int32)
+    f = harness().bh_regular_taken
+    f.argtypes = [C.c_void_p, C.c_long, C.c_void_p, C.c_double, C.c_double, C.c_double, C.c_void_p]
+    f.restype = C.c_long
+    n = f(z.ctypes.data, len(z), C.cast(arr, C.c_void_p), APERTURE, APERTURE, Po, taken.ctypes.data)
+    assert n == taken.sum()
+    if not has:
+        assert n == 0
+        return
+    assert taken[:48].all()
+    out = (~np.isfinite(z[:, [0, 1, 2, 3, 5]]).all(1)) | (np.abs(z[:, 3]) > 0.0125) | (z[:, 5] < -0.126) | (
+        z[:, 5] > 0.2501) | (np.abs(z[:, 0]) > APERTURE + 1e-4) | (np.abs(z[:, 2]) > APERTURE + 1e-4)
+    assert out.sum() > 20 and not taken[out].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(ELEMENTS))
+def test_gpu_matches_oracle(ehlib, name):
+    rows = np.concatenate([particles()] * 3)
+    rows[:, 6] = np.arange(1, len(rows) + 1)
+    beam = tracking.Beam(rows)
+    n, _, _ = tracking.track(beam, line(name), 2, Po, mode="fused", turns_per_launch=2)
+    got = beam.download()
+    beam.free()
+    ref, nref, _, _ = oracle.do_tracking(rows, line(name), 2, Po)
+    assert n == nref
+    check(got, ref, name)
