@@ -352,6 +352,12 @@ static long build_multipole(eh_desc *d, const EH_ELEMENT_LIST *e, const eh_ctx &
   if (!expand && mdrift != 0 && !d->ap_rtilt && !d->ell_any && d->mp_order[0] && !d->mp_order[1] && !d->mp_order[2] &&
       !skew[0])
     d->regular = d->mp_order[0];
+  d->reg_nsl = d->nslices;
+  d->reg_nsub = nsub;
+  for (int k = 0; k < 2; k++) {
+    d->reg_h[k] = d->dsh[k];
+    d->reg_k[k] = d->kick[k][0];
+  }
   return EH_OK;
 }
 
@@ -577,6 +583,12 @@ static long build_csbend(eh_desc *d, const EH_CSBEND *cb, const eh_ctx &c, std::
   }
   d->csb_dzl = cb->nSlices * s;
   d->regular = csb_regular(*d);
+  d->reg_nsl = cb->nSlices;
+  d->reg_nsub = nsub;
+  for (int k = 0; k < 2; k++) {
+    d->reg_h[k] = d->csb_dshr[k];
+    d->reg_k[k] = d->csb_ds[k];
+  }
   d->csb_edge1 = (cb->edgeFlags & EH_BEND_EDGE1_EFFECTS) && cb->edge1_effects >= 1;
   d->csb_edge2 = (cb->edgeFlags & EH_BEND_EDGE2_EFFECTS) && cb->edge2_effects >= 1;
   d->csb_esimple1 = d->csb_edge1 && cb->edge1_effects == 3;
@@ -823,7 +835,29 @@ static double elem_length(const EH_ELEMENT_LIST *e) {
   return *(const double *)e->p_elem;
 }
 
+static long build_element(eh_desc *d, const EH_ELEMENT_LIST *e, const eh_ctx &c, std::vector<eh_fterm> &pool);
+
+/* the head's limits: what the sweeps after the element clear without a look at
+ * their kind (a plain MAXAMP's limits, or every finite coordinate where there is
+ * none; nothing for elliptical ones), and the in-element limits */
+static void head_limits(eh_desc *d) {
+  for (int pi = 0; pi < 2; pi++) {
+    const bool on = d->post_ap[pi] != 0;
+    d->sw_x[pi] = d->post_ell[pi] ? -1.0 : on && d->post_xmax[pi] > 0 ? d->post_xmax[pi] : EH_DBL_MAX;
+    d->sw_y[pi] = d->post_ell[pi] ? -1.0 : on && d->post_ymax[pi] > 0 ? d->post_ymax[pi] : EH_DBL_MAX;
+    d->reg_apx[pi] = d->ap_xmax[pi] > 0 ? d->ap_xmax[pi] : 0x1p60;
+    d->reg_apy[pi] = d->ap_ymax[pi] > 0 ? d->ap_ymax[pi] : 0x1p60;
+  }
+}
+
 static long build_desc(eh_desc *d, const EH_ELEMENT_LIST *e, const eh_ctx &c, std::vector<eh_fterm> &pool) {
+  long r = build_element(d, e, c, pool);
+  if (r >= 0)
+    head_limits(d);
+  return r;
+}
+
+static long build_element(eh_desc *d, const EH_ELEMENT_LIST *e, const eh_ctx &c, std::vector<eh_fterm> &pool) {
   std::memset(d, 0, sizeof *d);
   d->type = e->type;
   d->counted = !(e->type == EH_T_MARK || e->type == EH_T_MAXAMP);
@@ -1415,12 +1449,15 @@ __device__ __forceinline__ void track_span(eh_p6 &p, bool &alive, const eh_pos *
                                            const eh_fterm *__restrict__ terms, int nelem, int p0, int e0, int p1,
                                            int e1, int32_t &lcode, unsigned long long &units) {
   int pp = p0, ee = e0;
+  int64_t next_off = pos[ee < nelem ? ee : 0].off;
   while (pp < p1 || (pp == p1 && ee < e1)) {
     const unsigned long long live = __ballot(alive);
     if (live == 0)
       break;
     const eh_pos *q = pos + ee;
-    const eh_desc *d = (const eh_desc *)((const char *)pos + q->off);
+    const eh_desc *d = (const eh_desc *)((const char *)pos + next_off);
+    /* the next position's offset arrives while this element is tracked */
+    next_off = pos[ee + 1 < nelem ? ee + 1 : 0].off;
     units += (unsigned long long)__popcll(live) * (unsigned)d->counted;
     if (alive) {
       int st = eh_apply_element_t<RAD>(p, *d, pp, terms, q->z);
@@ -1590,11 +1627,13 @@ __global__ void __launch_bounds__(EH_BLOCK) EH_TRACK_WAVES k_batch(eh_soa a, eh_
     /* descriptors of variant v: pool entries listed by desc_idx (uniform) */
     const int32_t *idx = bd.desc_idx + (long)v * nelem;
     int pp = p0, ee = e0;
+    int32_t next_idx = idx[ee < nelem ? ee : 0];
     while (pp < p1 || (pp == p1 && ee < e1)) {
       const unsigned long long live = __ballot(alive);
       if (live == 0)
         break;
-      const eh_desc *d = pool + __builtin_amdgcn_readfirstlane(idx[ee]);
+      const eh_desc *d = pool + __builtin_amdgcn_readfirstlane(next_idx);
+      next_idx = idx[ee + 1 < nelem ? ee + 1 : 0]; /* as in track_span */
       units += (unsigned long long)__popcll(live) * (unsigned)d->counted;
       if (alive) {
         int st = eh_apply_element_t<RAD>(p, *d, pp, terms, d->zpos);
@@ -2794,8 +2833,10 @@ static long track_fused(eh_beam *b, EH_ELEMENT_LIST *bl, long ne, long n_passes,
     long r2 = build_desc(&hd[ie], bl + ie, c, pool);
     /* an element followed by a matching: the reference sweeps its MAXAMP after
      * the matching, so the sweep runs on the host side after it */
-    if (r2 >= 0 && stop_after[ie])
+    if (r2 >= 0 && stop_after[ie]) {
       hd[ie].post_ap[0] = hd[ie].post_ap[1] = 0;
+      head_limits(&hd[ie]);
+    }
     return r2;
   };
   /* initial NaN sweep, src/do_tracking.c:478-483 */

@@ -123,17 +123,17 @@ EH_HD double eh_reg_asin(double x) {
 /* the field of a bend that has a gradient and nothing else, from the nine terms
  * of its dense block in the order of eh_csb_fields_dense; 0 + c y is one fma */
 struct eh_grad_field {
-  double y1, y2c, y3, y4, x1, x1y2, x1y3, x2y2, c0;
+  double c0, y1, y2, y3, y4, x1, x1y2, x1y3, x2y2;
 };
 
 EH_HD eh_grad_field eh_grad_load(const eh_fterm *__restrict__ cx, const eh_fterm *__restrict__ cy) {
-  return {cx[1].coef, cy[2].coef, cx[3].coef, cy[4].coef, cy[5].coef, cy[7].coef, cx[8].coef, cy[12].coef, cy[0].coef};
+  return {cy[0].coef, cx[1].coef, cy[2].coef, cx[3].coef, cy[4].coef, cy[5].coef, cy[7].coef, cx[8].coef, cy[12].coef};
 }
 
 EH_HD void eh_grad_eval(const eh_grad_field &c, double x, double y, double &Fx, double &Fy) {
   const double y2 = y * y, y3 = y2 * y, y4 = y3 * y;
   Fx = eh_fma(c.y1, y, 0.0);
-  Fy = c.c0 + c.y2c * y2;
+  Fy = c.c0 + c.y2 * y2;
   Fx += c.y3 * y3;
   Fy += c.y4 * y4;
   Fy += c.x1 * x;
@@ -157,7 +157,7 @@ EH_HD eh_reg_slopes eh_reg_m2s(double qx, double qy, double b1s, double rh, doub
 }
 
 /* zero, or far above underflow */
-EH_HD bool eh_reg_sized(double ax) { return ax >= EH_REG_QMIN || ax == 0; }
+EH_HD bool eh_reg_sized(double ax) { return (ax >= EH_REG_QMIN) | (ax == 0); }
 
 /* the field sums of one kick of order N, eh_mkick's terms and order (0 + v is
  * v + 0, one fma where v is a product) */
@@ -189,7 +189,9 @@ EH_HD bool eh_mult_regular(const eh_desc &d, int pi, double &x_, double &xp_, do
                            double dp) {
   double x = x_, y = y_, s = 0;
   const double mdx = d.mdx, mdy = d.mdy;
-  const double apx = d.ap_xmax[pi] > 0 ? d.ap_xmax[pi] : 0x1p60, apy = d.ap_ymax[pi] > 0 ? d.ap_ymax[pi] : 0x1p60;
+  const double apx = d.reg_apx[pi], apy = d.reg_apy[pi];
+  const double h0 = d.reg_h[0], h1 = d.reg_h[1], k0 = d.reg_k[0], k1 = d.reg_k[1];
+  const bool steering = d.has_xkick || d.has_ykick;
   const double b1 = 1 + dp;
   bool bad = !(b1 >= EH_REG_B1_MIN && b1 <= EH_REG_B1_MAX && eh_fabs(x) <= 10.0 && eh_fabs(y) <= 10.0 &&
                eh_fabs(xp_) <= EH_REG_QMAX && eh_fabs(yp_) <= EH_REG_QMAX && eh_reg_sized(eh_fabs(xp_)) &&
@@ -211,11 +213,13 @@ EH_HD bool eh_mult_regular(const eh_desc &d, int pi, double &x_, double &xp_, do
     qy = eh_reg_div(b1 * yp_, w, yw);
   }
   eh_reg_slopes v = eh_reg_m2s(qx, qy, b1s, rh, rh2);
-  const int nsl = d.nslices, nsub = d.nsub;
+  const int nsl = d.reg_nsl, nsub = d.reg_nsub;
   for (int ik = 0; ik < nsl; ik++) {
-    bad = bad || !(eh_fabs(x + mdx) <= apx && eh_fabs(y + mdy) <= apy);
+    bad |= !((eh_fabs(x + mdx) <= apx) & (eh_fabs(y + mdy) <= apy));
     for (int step = 0; step < nsub; step++) {
-      const double dsh = d.dsh[step];
+      double dsh = step == 1 || step == 2 ? h1 : h0;
+      if (nsub == 8)
+        dsh = d.dsh[step];
       x += v.xp * dsh;
       y += v.yp * dsh;
       const double a2 = 1 + eh_sqr(v.xp) + eh_sqr(v.yp);
@@ -225,28 +229,34 @@ EH_HD bool eh_mult_regular(const eh_desc &d, int pi, double &x_, double &xp_, do
         break;
       double Fx, Fy;
       eh_reg_mfield<ORDER>(x, y, Fx, Fy);
-      const double K = d.kick[step][0];
+      double K = step == 1 ? k1 : k0;
+      if (nsub == 8)
+        K = d.kick[step][0];
       qx -= K * Fy;
       qy += K * Fx;
-      if (d.has_xkick) { /* eh_mkick<0>: the other plane gains a signed zero */
-        qx -= d.xk[step];
-        qy += d.xk[step] * 0.0;
-      }
-      if (d.has_ykick) {
-        qx -= d.yk[step] * 0.0;
-        qy -= d.yk[step];
+      if (steering) {
+#if defined(__HIP_DEVICE_COMPILE__)
+        __asm__ volatile(""); /* a scalar branch, not selects */
+#endif
+        /* eh_mkick<0>: the other plane gains a signed zero */
+        if (d.has_xkick) {
+          qx -= d.xk[step];
+          qy += d.xk[step] * 0.0;
+        }
+        if (d.has_ykick) {
+          qx -= d.yk[step] * 0.0;
+          qy -= d.yk[step];
+        }
       }
       const double ax = eh_fabs(qx), ay = eh_fabs(qy);
-      bad = bad || !(ax <= EH_REG_QMAX && ay <= EH_REG_QMAX);
-      if (!(ax >= EH_REG_QMIN && ay >= EH_REG_QMIN))
-        bad = bad || !(eh_reg_sized(ax) && eh_reg_sized(ay));
+      bad |= !((ax <= EH_REG_QMAX) & (ay <= EH_REG_QMAX) & eh_reg_sized(ax) & eh_reg_sized(ay));
       /* the radiation block's division and multiplication by 1 + delta */
       qx = eh_reg_div(qx, b1, rh) * b1;
       qy = eh_reg_div(qy, b1, rh) * b1;
       v = eh_reg_m2s(qx, qy, b1s, rh, rh2);
     }
   }
-  bad = bad || !(eh_fabs(x + mdx) <= apx && eh_fabs(y + mdy) <= apy && eh_fabs(x) <= 10.0 && eh_fabs(y) <= 10.0);
+  bad |= !((eh_fabs(x + mdx) <= apx) & (eh_fabs(y + mdy) <= apy) & (eh_fabs(x) <= 10.0) & (eh_fabs(y) <= 10.0));
   if (bad)
     return false;
   x_ = x;
@@ -266,21 +276,38 @@ EH_HD bool eh_mult_regular_n(const eh_desc &d, int pi, double &x, double &xp, do
   return eh_mult_regular<3>(d, pi, x, xp, y, yp, s, dp);
 }
 
-/* integrate_csbend_ordn without losses for a regular particle: X, QX, Y, QY and
- * the path `dist` advance through the bend if it returns true and are left alone
- * otherwise.  FIELD as eh_desc.regular. */
+/* integrate_csbend_ordn without losses for a regular particle, slopes to momenta
+ * before it and back after it: X, xp, Y, yp and the path `dist` advance through
+ * the bend if it returns true and are left alone otherwise.  FIELD as
+ * eh_desc.regular. */
 template <int FIELD>
-EH_HD bool eh_csb_regular(const eh_desc &d, int pi, const eh_fterm *__restrict__ terms, double b1, double rh,
-                          double &X_, double &QX_, double &Y_, double &QY_, double &dist_) {
-  double X = X_, QX = QX_, Y = Y_, QY = QY_, dist = 0;
+EH_HD bool eh_csb_regular(const eh_desc &d, int pi, const eh_fterm *__restrict__ terms, double b1, double &X_,
+                          double &xp_, double &Y_, double &yp_, double &dist_) {
+  double X = X_, QX, Y = Y_, QY, dist = 0;
+  bool bad = !(b1 >= EH_REG_B1_MIN && b1 <= EH_REG_B1_MAX && eh_fabs(xp_) <= EH_REG_QMAX &&
+               eh_fabs(yp_) <= EH_REG_QMAX && eh_reg_sized(eh_fabs(yp_)));
+#if defined(__HIP_DEVICE_COMPILE__)
+  if (__ballot(!bad) == 0)
+    return false;
+#else
+  if (bad)
+    return false;
+#endif
   const double rho0 = d.rho0, rho_a = d.rho_actual, r0h = d.rho0_rh, rah = d.rhoa_rh;
-  const double apx = d.ap_xmax[pi] > 0 ? d.ap_xmax[pi] : 0x1p60, apy = d.ap_ymax[pi] > 0 ? d.ap_ymax[pi] : 0x1p60;
-  const double b1s = b1 * b1, rh2 = rh * rh;
+  const double apx = d.reg_apx[pi], apy = d.reg_apy[pi];
+  const double h0 = d.reg_h[0], h1 = d.reg_h[1], k0 = d.reg_k[0], k1 = d.reg_k[1];
+  const double b1s = b1 * b1, rh = 1.0 / b1, rh2 = rh * rh;
   eh_grad_field gf;
   if constexpr (FIELD == 2)
     gf = eh_grad_load(terms + d.csb_dx0, terms + d.csb_dy0);
-  bool bad = !(b1 >= EH_REG_B1_MIN && b1 <= EH_REG_B1_MAX && eh_fabs(QY) <= EH_REG_QMAX &&
-               (eh_fabs(QY) >= EH_REG_QMIN || QY == 0));
+  {
+    const double u = eh_sqr(xp_) + eh_sqr(yp_);
+    double w, yw;
+    eh_reg_root(1 + eh_sqr(xp_) + eh_sqr(yp_), -u, 1.0, w, yw);
+    const double c = eh_reg_div(b1, w, yw);
+    QX = xp_ * c;
+    QY = yp_ * c;
+  }
   /* f and 1 / f depend on QY alone, which drifts leave unchanged: formed at
    * entry and after every kick */
   double f, y;
@@ -288,10 +315,10 @@ EH_HD bool eh_csb_regular(const eh_desc &d, int pi, const eh_fterm *__restrict__
     const double q2 = QY * QY;
     eh_reg_root(b1s - q2, q2 * rh2, rh, f, y);
   }
-  const int nsl = d.csb_nslices, nsub = d.nsub;
+  const int nsl = d.reg_nsl, nsub = d.reg_nsub;
   for (int i = 0; i < nsl; i++) {
-    bad = bad || !(eh_fabs(X) <= apx && eh_fabs(Y) <= apy && eh_fabs(QX) <= EH_REG_QXMAX &&
-                   eh_fabs(QX) >= EH_REG_QMIN);
+    bad |= !((eh_fabs(X) <= apx) & (eh_fabs(Y) <= apy) & (eh_fabs(QX) <= EH_REG_QXMAX) &
+             (eh_fabs(QX) >= EH_REG_QMIN));
 #if defined(__HIP_DEVICE_COMPILE__)
     if (__ballot(!bad) == 0)
       break;
@@ -302,8 +329,11 @@ EH_HD bool eh_csb_regular(const eh_desc &d, int pi, const eh_fterm *__restrict__
     for (int j = 0; j < nsub; j++) {
       const double sin_phi = eh_reg_div(QX, f, y);
       const double phi = eh_reg_asin(sin_phi);
-      const double ang = d.csb_dshr[j] + phi;
-      bad = bad || !(eh_fabs(ang) < 0x1p-4); /* the short series of eh_sincos */
+      double th = j == 1 || j == 2 ? h1 : h0;
+      if (nsub == 8)
+        th = d.csb_dshr[j];
+      const double ang = th + phi;
+      bad |= !(eh_fabs(ang) < 0x1p-4); /* the short series of eh_sincos */
       const double sine = eh_sin_poly(ang), cosi = eh_cos_poly(ang);
       const double yc = eh_reg_recip1(cosi);
       const double tang = eh_reg_div(sine, cosi, yc);
@@ -317,7 +347,10 @@ EH_HD bool eh_csb_regular(const eh_desc &d, int pi, const eh_fterm *__restrict__
       X = rho0 * (fr - 1) + fr * X;
       if (j == nsub - 1)
         break;
-      const double u = d.csb_ds[j] * (1 + eh_reg_div(X, rho0, r0h));
+      double ds = j == 1 ? k1 : k0;
+      if (nsub == 8)
+        ds = d.csb_ds[j];
+      const double u = ds * (1 + eh_reg_div(X, rho0, r0h));
       double Fx = 0, Fy = 1;
       if constexpr (FIELD == 2)
         eh_grad_eval(gf, X, Y, Fx, Fy);
@@ -329,9 +362,8 @@ EH_HD bool eh_csb_regular(const eh_desc &d, int pi, const eh_fterm *__restrict__
       /* a momentum far above underflow has lost nothing to an inexact tiny
        * kick; a particle in the mid-plane keeps QY = 0 exactly */
       const double ax = eh_fabs(QX), ay = eh_fabs(QY);
-      bad = bad || !(ax <= EH_REG_QXMAX && ay <= EH_REG_QMAX);
-      if (!(ax >= EH_REG_QMIN && ay >= EH_REG_QMIN))
-        bad = bad || !(ax >= EH_REG_QMIN && QY == 0 && ny == 0);
+      bad |= !((ax <= EH_REG_QXMAX) & (ay <= EH_REG_QMAX) & (ax >= EH_REG_QMIN) &
+               ((ay >= EH_REG_QMIN) | ((QY == 0) & (ny == 0))));
       /* the radiation block's division and multiplication by 1 + delta */
       QX = eh_reg_div(QX, b1, rh) * b1;
       QY = eh_reg_div(QY, b1, rh) * b1;
@@ -339,24 +371,27 @@ EH_HD bool eh_csb_regular(const eh_desc &d, int pi, const eh_fterm *__restrict__
       eh_reg_root(b1s - q2, q2 * rh2, rh, f, y);
     }
   }
-  bad = bad || !(eh_fabs(X) <= apx && eh_fabs(Y) <= apy);
+  bad |= !((eh_fabs(X) <= apx) & (eh_fabs(Y) <= apy) & (eh_fabs(QX) <= EH_REG_QMAX));
   if (bad)
     return false;
+  const double x2 = QX * QX, y2 = QY * QY;
+  eh_reg_root(b1s - x2 - y2, (x2 + y2) * rh2, rh, f, y);
+  const double c = eh_reg_div(1.0, f, y);
   X_ = X;
-  QX_ = QX;
+  xp_ = QX * c;
   Y_ = Y;
-  QY_ = QY;
+  yp_ = QY * c;
   dist_ = dist;
   return true;
 }
 
-EH_HD bool eh_csb_regular_n(const eh_desc &d, int pi, const eh_fterm *__restrict__ terms, double b1, double rh,
-                            double &X, double &QX, double &Y, double &QY, double &dist) {
+EH_HD bool eh_csb_regular_n(const eh_desc &d, int pi, const eh_fterm *__restrict__ terms, double b1, double &X,
+                            double &xp, double &Y, double &yp, double &dist) {
   if (d.regular == 2)
-    return eh_csb_regular<2>(d, pi, terms, b1, rh, X, QX, Y, QY, dist);
+    return eh_csb_regular<2>(d, pi, terms, b1, X, xp, Y, yp, dist);
   if (d.regular == 1)
-    return eh_csb_regular<1>(d, pi, terms, b1, rh, X, QX, Y, QY, dist);
-  return eh_csb_regular<3>(d, pi, terms, b1, rh, X, QX, Y, QY, dist);
+    return eh_csb_regular<1>(d, pi, terms, b1, X, xp, Y, yp, dist);
+  return eh_csb_regular<3>(d, pi, terms, b1, X, xp, Y, yp, dist);
 }
 
 #endif

@@ -390,9 +390,7 @@ extern "C" long bh_regular_taken(const double *z, long n, const EH_ELEMENT_LIST 
     const double b1 = 1 + z[6 * i + 5];
     taken[i] = 0;
     if (d.regular && d.type == EH_T_CSBEND) {
-      const double f = b1 / eh_sqrt(1 + xp * xp + yp * yp);
-      double QX = xp * f, QY = yp * f;
-      taken[i] = eh_csb_regular_n(d, 0, terms.data(), b1, 1.0 / b1, x, QX, y, QY, s);
+      taken[i] = eh_csb_regular_n(d, 0, terms.data(), b1, x, xp, y, yp, s);
     } else if (d.regular) {
       taken[i] = eh_mult_regular_n(d, 0, x, xp, y, yp, s, z[6 * i + 5]);
     }
