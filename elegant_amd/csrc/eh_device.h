@@ -83,6 +83,9 @@ typedef struct {
    * slice, 1 for the inner ones (the integrators of order 2 and 4 are symmetric;
    * order 6 reads the tables below); bends: angles and kick lengths */
   double reg_h[2], reg_k[2];
+  /* with SYNCH_RAD, multipoles (order 2 and 4): kick fractions and their
+   * reciprocals, the reciprocal of the slice drift and the steering terms over it */
+  double reg_kf[2], reg_ikf[2], reg_idrift, reg_rxk, reg_ryk;
   union {
     struct { /* bends */
       double rho0, rho_actual;
@@ -637,8 +640,9 @@ EH_HD void eh_mface2(eh_p6 &p, const eh_desc &d, bool s_too) {
   }
 }
 
+template <bool RAD>
 EH_HD bool eh_mult_regular_n(const eh_desc &d, int pi, double &x, double &xp, double &y, double &yp, double &s,
-                             double dp);
+                             double &dp);
 
 /* KQUAD/KSEXT/KOCT/KQUSE: multipole_tracking2 (src/multipole.c:660-1084) for one
  * particle, including the misalignment passes around the particle loop (method 0,
@@ -665,10 +669,8 @@ EH_HD int eh_multipole_t(eh_p6 &p, const eh_desc &d, int pi, const double *__res
   bool lost = false, entry = false;
   int how = 0; /* 0: coord untouched, 1: x,y written, 2: all written */
   bool regular = false;
-  if constexpr (!RAD) {
-    if (d.regular)
-      regular = eh_mult_regular_n(d, pi, x, xp, y, yp, s, dp);
-  }
+  if (d.regular)
+    regular = eh_mult_regular_n<RAD>(d, pi, x, xp, y, yp, s, dp);
   if (regular) {
     how = 2;
   } else if (eh_isnan(x) || eh_isnan(xp) || eh_isnan(y) || eh_isnan(yp) || eh_fabs(x) > 10.0 || eh_fabs(y) > 10.0 ||
@@ -1412,10 +1414,8 @@ EH_HD bool eh_csbend_t(eh_p6 &p, const eh_desc &d, int pi, const eh_fterm *__res
   const double b1 = 1 + DP;
   double dist = 0, dz_lost = 0;
   bool lost = false, regular = false;
-  if constexpr (!RAD) {
-    if (d.regular)
-      regular = eh_csb_regular_n(d, pi, terms, b1, X, QX, Y, QY, dist);
-  }
+  if (d.regular)
+    regular = eh_csb_regular_n<RAD>(d, pi, terms, X, QX, Y, QY, DP, dist);
   /* integrate_csbend_ordn; the reciprocal pair of 1 + DPoP is for the radiation
    * block's round trip after each kick */
   double rh = 0, rl = 0;

@@ -350,8 +350,15 @@ static long build_multipole(eh_desc *d, const EH_ELEMENT_LIST *e, const eh_ctx &
   /* the regular path: one term, an untilted rectangular aperture, a length (the
    * radiation block's round trip runs) and the exact Hamiltonian */
   if (!expand && mdrift != 0 && !d->ap_rtilt && !d->ell_any && d->mp_order[0] && !d->mp_order[1] && !d->mp_order[2] &&
-      !skew[0])
+      !skew[0] && !(d->rad && nsub == 8))
     d->regular = d->mp_order[0];
+  for (int k = 0; k < 2; k++) {
+    d->reg_kf[k] = kickFrac[k];
+    d->reg_ikf[k] = 1.0 / kickFrac[k];
+  }
+  d->reg_idrift = 1.0 / mdrift;
+  d->reg_rxk = d->rad_xk / mdrift;
+  d->reg_ryk = d->rad_yk / mdrift;
   d->reg_nsl = d->nslices;
   d->reg_nsub = nsub;
   for (int k = 0; k < 2; k++) {

@@ -387,12 +387,14 @@ extern "C" long bh_regular_taken(const double *z, long n, const EH_ELEMENT_LIST 
   long count = 0;
   for (long i = 0; i < n; i++) {
     double x = z[6 * i], xp = z[6 * i + 1], y = z[6 * i + 2], yp = z[6 * i + 3], s = 0;
-    const double b1 = 1 + z[6 * i + 5];
+    double dp = z[6 * i + 5];
     taken[i] = 0;
     if (d.regular && d.type == EH_T_CSBEND) {
-      taken[i] = eh_csb_regular_n(d, 0, terms.data(), b1, x, xp, y, yp, s);
+      taken[i] = d.rad ? eh_csb_regular_n<true>(d, 0, terms.data(), x, xp, y, yp, dp, s)
+                       : eh_csb_regular_n<false>(d, 0, terms.data(), x, xp, y, yp, dp, s);
     } else if (d.regular) {
-      taken[i] = eh_mult_regular_n(d, 0, x, xp, y, yp, s, z[6 * i + 5]);
+      taken[i] = d.rad ? eh_mult_regular_n<true>(d, 0, x, xp, y, yp, s, dp)
+                       : eh_mult_regular_n<false>(d, 0, x, xp, y, yp, s, dp);
     }
     count += taken[i];
   }

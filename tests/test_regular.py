@@ -39,6 +39,15 @@ ELEMENTS = {
     "quad_off": (Element("Q", "KQUAD", L=0.25, K1=0.0, N_KICKS=8), False),
     "sext": (Element("X", "KSEXT", L=0.2, K2=-25.0, N_KICKS=4), True),
     "sext_k1": (Element("X", "KSEXT", L=0.2, K2=-25.0, K1=0.1, N_KICKS=4), False),
+    "bend_rad": (Element("B", "CSBEND", SYNCH_RAD=1, **BEND), True),
+    "bend_k1_rad_edges": (Element("B", "CSBEND", K1=0.5, SYNCH_RAD=1, **{
+        **BEND, "EDGE1_EFFECTS": 1, "EDGE2_EFFECTS": 1, "E1": 0.015, "E2": 0.015, "HGAP": 0.01}), True),
+    "bend_k2_rad": (Element("B", "CSBEND", K2=4.0, SYNCH_RAD=1, **BEND), True),
+    "quad_rad": (Element("Q", "KQUAD", L=0.25, K1=2.9, N_KICKS=8, SYNCH_RAD=1, HKICK=1e-5, VKICK=-2e-5, DX=1e-4),
+                 True),
+    "quad_rad_order6": (Element("Q", "KQUAD", L=0.25, K1=2.9, N_KICKS=6, SYNCH_RAD=1, INTEGRATION_ORDER=6), False),
+    "sext_rad": (Element("X", "KSEXT", L=0.2, K2=-25.0, N_KICKS=4, SYNCH_RAD=1), True),
+    "oct_rad": (Element("O", "KOCT", L=0.2, K3=-1000.0, SYNCH_RAD=1), True),
     "oct": (Element("O", "KOCT", L=0.2, K3=-1000.0), True),
 }
 APERTURE = 0.02
@@ -107,7 +116,7 @@ def test_host_build_matches_oracle(name):
     where = ref[:, 6].astype(int) - 1
     got[:, :6] = out6[where]
     # the position of a loss at entry, or in an element with an exit offset, is settled on download
-    settled = (lpass[where] != -1) & ((lpass[where] & 0x40000000 != 0) | ("DZ" in ELEMENTS[name][0].params))
+    settled = (lpass[where] != -1) & ((lpass[where] & 0x40000000 != 0) | ("DX" in ELEMENTS[name][0].params))
     got[settled, 4] = ref[settled, 4]
     check(got, ref, name)
 
