@@ -129,14 +129,14 @@ EH_HD double eh_reg_asin(double x) {
 #endif
   {
     double p = EH_ASIN_7;
-    p = EH_ASIN_6 + z * p;
-    p = EH_ASIN_5 + z * p;
-    p = EH_ASIN_4 + z * p;
+    p = eh_horner(z, p, EH_ASIN_6);
+    p = eh_horner(z, p, EH_ASIN_5);
+    p = eh_horner(z, p, EH_ASIN_4);
     q = longer ? p : q;
   }
-  q = EH_ASIN_3 + z * q;
-  q = EH_ASIN_2 + z * q;
-  q = EH_ASIN_1 + z * q;
+  q = eh_horner(z, q, EH_ASIN_3);
+  q = eh_horner(z, q, EH_ASIN_2);
+  q = eh_horner(z, q, EH_ASIN_1);
   return eh_fma(x * z, q, x);
 }
 
