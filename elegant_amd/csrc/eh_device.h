@@ -195,6 +195,8 @@ typedef struct {
   int32_t adj_anchor;              /* slot of the stored entry state (RF cavity), -1 if none */
   double adj_kfac[EH_MAXSUB];      /* d kick[step][0] / d strength */
   double adj_sin_dshr[EH_MAXSUB];  /* sin of the CSBEND sub-step angles */
+  double adj_vers_dshr[EH_MAXSUB]; /* 1 - cos of them */
+  double adj_per_k1;               /* gradient bends: d field / d K1 over the field's gradient terms */
   /* bends as parameters: adj_pk is the slot of K1, adj_pfse that of FSE; the
    * field per unit K1 and per unit FSE as term lists (i, j, coefficient) in
    * the term pool; adj_fse1 = 1 / (1 + FSE + FSE_DIPOLE), the relative change

@@ -586,6 +586,7 @@ static long build_csbend(eh_desc *d, const EH_CSBEND *cb, const eh_ctx &c, std::
     d->csb_dsh[j] = s * driftFrac[j];
     d->csb_dshr[j] = d->csb_dsh[j] / rho0;
     d->adj_sin_dshr[j] = eh_sin(d->csb_dshr[j]);
+    d->adj_vers_dshr[j] = 2 * eh_sqr(eh_sin(0.5 * d->csb_dshr[j]));
     d->csb_ds[j] = s * kickFrac[j];
   }
   d->csb_dzl = cb->nSlices * s;
@@ -1680,13 +1681,43 @@ static long ensure_desc(eh_beam *b, long n) {
   return EH_OK;
 }
 
+/* point a bend at the first of the field-term blocks equal to its own (every bend
+ * appends its block to the pool), so that bends that differ only in where their
+ * terms lie get equal descriptors */
+typedef std::unordered_map<std::string, int32_t> eh_term_blocks;
+
+static void share_terms(eh_desc &d, const std::vector<eh_fterm> &pool, eh_term_blocks &blocks) {
+  if (d.type != EH_T_CSBEND)
+    return;
+  const int32_t from = d.csb_dense ? d.csb_dx0 : d.csb_fx0;
+  int32_t to = d.csb_fy0 + d.csb_nfy;
+  /* the adjoint's lists of a bend follow its field terms */
+  int32_t *adj0[4] = {&d.adj_dk_fx0, &d.adj_dk_fy0, &d.adj_df_fx0, &d.adj_df_fy0};
+  const int32_t adjn[4] = {d.adj_dk_nfx, d.adj_dk_nfy, d.adj_df_nfx, d.adj_df_nfy};
+  for (int k = 0; k < 4; k++)
+    to = adjn[k] ? std::max(to, *adj0[k] + adjn[k]) : to;
+  if (from < 0 || to > (int32_t)pool.size() || from >= to)
+    return;
+  std::string key(reinterpret_cast<const char *>(pool.data() + from), sizeof(eh_fterm) * (size_t)(to - from));
+  const int32_t shift = blocks.emplace(std::move(key), from).first->second - from;
+  d.csb_fx0 += shift;
+  d.csb_fy0 += shift;
+  if (d.csb_dense) {
+    d.csb_dx0 += shift;
+    d.csb_dy0 += shift;
+  }
+  for (int k = 0; k < 4; k++)
+    *adj0[k] = adjn[k] ? *adj0[k] + shift : 0;
+}
+
 /* the line's descriptors for the fused kernel, in one buffer: a table of
  * positions (eh_pos: z pair, byte offset of the descriptor) followed by the
  * distinct descriptors.  Positions whose descriptors are equal apart from their
  * z share one, so a ring of identical cells reads a few dozen descriptors
  * instead of one per position. */
-static long upload_fused_descs(eh_beam *b, const std::vector<eh_desc> &hd) {
+static long upload_fused_descs(eh_beam *b, const std::vector<eh_desc> &hd, const std::vector<eh_fterm> &pool) {
   const long ne = (long)hd.size();
+  eh_term_blocks blocks;
   std::vector<eh_desc> uniq;
   std::vector<eh_pos> pos(ne);
   std::unordered_map<std::string, int64_t> seen;
@@ -1698,6 +1729,7 @@ static long upload_fused_descs(eh_beam *b, const std::vector<eh_desc> &hd) {
     pos[ie].z[1] = k.zpos[1];
     pos[ie].pad_ = 0;
     k.zpos[0] = k.zpos[1] = 0;
+    share_terms(k, pool, blocks);
     std::string key(reinterpret_cast<const char *>(&k), sizeof k);
     auto it = seen.find(key);
     if (it == seen.end()) {
@@ -2891,7 +2923,7 @@ static long track_fused(eh_beam *b, EH_ELEMENT_LIST *bl, long ne, long n_passes,
     if (r < 0)
       return r;
   }
-  r = upload_fused_descs(b, hd);
+  r = upload_fused_descs(b, hd, pool);
   if (r < 0)
     return r;
   r = upload_terms(b, pool);
@@ -2938,7 +2970,7 @@ static long track_fused(eh_beam *b, EH_ELEMENT_LIST *bl, long ne, long n_passes,
       if (r2 < 0)
         return r2;
     }
-    return upload_fused_descs(b, hd);
+    return upload_fused_descs(b, hd, pool);
   };
   int p = 0, e = 0;
   if (dynamic) {
@@ -2973,7 +3005,7 @@ static long track_fused(eh_beam *b, EH_ELEMENT_LIST *bl, long ne, long n_passes,
         if (r2 < 0)
           return r2;
       }
-      long r2 = upload_fused_descs(b, hd);
+      long r2 = upload_fused_descs(b, hd, pool);
       if (r2 < 0)
         return r2;
       return upload_terms(b, pool);
@@ -3012,7 +3044,7 @@ static long track_fused(eh_beam *b, EH_ELEMENT_LIST *bl, long ne, long n_passes,
         r = build(e);
         if (r < 0)
           return r;
-        r = upload_fused_descs(b, hd);
+        r = upload_fused_descs(b, hd, pool);
         if (r < 0)
           return r;
       }
@@ -3045,7 +3077,7 @@ static long track_fused(eh_beam *b, EH_ELEMENT_LIST *bl, long ne, long n_passes,
           if (r < 0)
             return r;
           if (m->elliptical) { /* the per-element sweep used descriptor slot 0 */
-            r = upload_fused_descs(b, hd);
+            r = upload_fused_descs(b, hd, pool);
             if (r < 0)
               return r;
           }
@@ -3101,7 +3133,7 @@ static long track_fused(eh_beam *b, EH_ELEMENT_LIST *bl, long ne, long n_passes,
         if (r < 0)
           return r;
       }
-      r = upload_fused_descs(b, hd);
+      r = upload_fused_descs(b, hd, pool);
       if (r < 0)
         return r;
       r = upload_terms(b, pool);
@@ -4042,23 +4074,67 @@ extern "C" long eh_batch_track(eh_batch *b, EH_ELEMENT_LIST *const *beamlines, l
 
 #define EH_ADJ_BLOCK 64
 
+/* one position of a line: its z pair, the byte offset of its descriptor from the
+ * start of the table, its gradient slots (strength, DX, DY, FSE; -1 none) and its
+ * anchor slot.  Positions that differ only in these share one descriptor, as in
+ * the fused kernel: with a descriptor per position every wavefront read 3.8 MB per
+ * turn through its scalar cache, each line a miss. */
+struct eh_apos {
+  double z[2];
+  int64_t off;
+  int32_t slot[4];
+  int32_t anchor, pad_;
+};
+
+/* the table of all variants' positions followed by the distinct descriptors */
+static std::vector<char> adj_table(const std::vector<eh_desc> &hd, const std::vector<eh_fterm> &pool) {
+  std::vector<eh_apos> pos(hd.size());
+  std::vector<eh_desc> uniq;
+  std::unordered_map<std::string, int64_t> seen;
+  eh_term_blocks blocks;
+  const int64_t base = (int64_t)(sizeof(eh_apos) * hd.size());
+  for (size_t i = 0; i < hd.size(); i++) {
+    eh_desc k;
+    std::memcpy(&k, &hd[i], sizeof k);
+    pos[i] = {{k.zpos[0], k.zpos[1]}, 0, {k.adj_pk, k.adj_pdx, k.adj_pdy, k.adj_pfse}, k.adj_anchor, 0};
+    k.zpos[0] = k.zpos[1] = 0;
+    k.adj_anchor = -1;
+    /* the maps ask only whether there is a slot */
+    for (int32_t *s : {&k.adj_pk, &k.adj_pdx, &k.adj_pdy, &k.adj_pfse})
+      *s = *s >= 0 ? 0 : -1;
+    share_terms(k, pool, blocks);
+    std::string key(reinterpret_cast<const char *>(&k), sizeof k);
+    auto it = seen.find(key);
+    if (it == seen.end()) {
+      it = seen.emplace(std::move(key), base + (int64_t)(sizeof(eh_desc) * uniq.size())).first;
+      uniq.push_back(k);
+    }
+    pos[i].off = it->second;
+  }
+  std::vector<char> table((size_t)base + sizeof(eh_desc) * uniq.size());
+  std::memcpy(table.data(), pos.data(), (size_t)base);
+  std::memcpy(table.data() + base, uniq.data(), sizeof(eh_desc) * uniq.size());
+  return table;
+}
+
 /* forward over turns [t0, t1) for particles i < n in fixed rows; anchors (if
  * given) receive the entry state of element 0 (slot 0) and of each anchor
  * element (slot d.adj_anchor) for every turn, at index
  * ((t - t0) * n_anchor + slot) * 6 * a_ld + c * a_ld + i */
 __global__ void __launch_bounds__(EH_BLOCK) EH_TRACK_WAVES k_adj_fwd(double *z, long ld, int32_t *alive, long n,
-                                                       const eh_desc *__restrict__ descs,
+                                                       const eh_apos *__restrict__ table,
                                                        const eh_fterm *__restrict__ terms, int ne, int t0, int t1,
                                                        double *anchors, int n_anchor, long a_ld,
                                                        unsigned long long *units, const int32_t *cvar) {
   long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   bool in = i < n;
   /* lattice variants: rows come in 64-row chunks of one variant each (cvar),
-   * whose descriptors are the variant's block of ne; the chunk is the wavefront */
+   * whose positions are the variant's block of ne; the chunk is the wavefront */
+  const eh_apos *pos = table;
   if (cvar) {
     const long chunk = i >> 6;
     const int v = __builtin_amdgcn_readfirstlane(chunk < (n + 63) / 64 ? cvar[chunk] : 0);
-    descs += (long)v * ne;
+    pos += (long)v * ne;
   }
   bool live = in && alive[i];
   eh_p6 p = {0, 0, 0, 0, 0, 0};
@@ -4068,10 +4144,13 @@ __global__ void __launch_bounds__(EH_BLOCK) EH_TRACK_WAVES k_adj_fwd(double *z, 
   for (int t = t0; t < t1; t++) {
     if (__ballot(live) == 0)
       break;
+    int64_t next_off = pos[0].off;
     for (int e = 0; e < ne; e++) {
-      const eh_desc *d = descs + e;
+      const eh_apos *q = pos + e;
+      const eh_desc *d = (const eh_desc *)((const char *)table + next_off);
+      next_off = pos[e + 1 < ne ? e + 1 : 0].off; /* as in track_span */
       if (live) {
-        int slot = e == 0 ? 0 : d->adj_anchor;
+        int slot = e == 0 ? 0 : q->anchor;
         if (anchors && slot >= 0) {
           double *a = anchors + ((long)(t - t0) * n_anchor + slot) * 6 * a_ld + i;
           a[0] = p.x;
@@ -4082,7 +4161,7 @@ __global__ void __launch_bounds__(EH_BLOCK) EH_TRACK_WAVES k_adj_fwd(double *z, 
           a[5 * a_ld] = p.dp;
         }
         u += d->counted;
-        if (eh_apply_element_t<false>(p, *d, t, terms, d->zpos) >= 0)
+        if (eh_apply_element_t<false>(p, *d, t, terms, q->z) >= 0)
           live = false;
       }
     }
@@ -4108,10 +4187,36 @@ __global__ void k_adj_gather(const double *in, long ld, const int32_t *rows, lon
       out[c * m + i] = in[c * ld + rows[i]];
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
-  for (int off = 32; off > 0; off >>= 1)
-    v += __shfl_xor(v, off, 64);
+/* v of another lane through the data-parallel primitives, 0 where there is none */
+template <int CTRL, int ROWS> __device__ __forceinline__ double dpp_or_zero(double v) {
+  const uint64_t u = eh_bits(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, ROWS, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, ROWS, 0xf, true);
+  return eh_from_bits(((uint64_t)hi << 32) | lo);
+}
+
+/* the sum over the wavefront, in lane 63, in a fixed order: within rows of 16
+ * lanes by row_shr 1, 2, 4, 8, then row_bcast 15 and 31.  18 vector instructions;
+ * six exchanges through LDS (ds_bpermute) took about 1000 cycles, of which a
+ * reverse sweep pays one or more per parameter and turn. */
+__device__ __forceinline__ double wave_sum63(double v) {
+  v += dpp_or_zero<0x111, 0xf>(v);
+  v += dpp_or_zero<0x112, 0xf>(v);
+  v += dpp_or_zero<0x114, 0xf>(v);
+  v += dpp_or_zero<0x118, 0xf>(v);
+  v += dpp_or_zero<0x142, 0xa>(v);
+  v += dpp_or_zero<0x143, 0xc>(v);
   return v;
+}
+
+/* add the wavefront's sum of v to its slot (none if negative): one wavefront per
+ * block, so the order is the program's */
+__device__ __forceinline__ void add_slot(double *lds, int slot, double v) {
+  if (slot < 0)
+    return;
+  v = wave_sum63(v);
+  if (threadIdx.x == 63)
+    unsafeAtomicAdd(lds + slot, v);
 }
 
 __device__ __forceinline__ double wave_max(double v) {
@@ -4134,15 +4239,16 @@ __device__ __forceinline__ eh_p6 load_anchor(const double *anchors, long idx, lo
 __global__ void __launch_bounds__(EH_ADJ_BLOCK) __attribute__((amdgpu_waves_per_eu(3)))
 k_adj_bwd(double *zb, double *lam, long m, const int32_t *arow,
                                                            const double *__restrict__ anchors, int n_anchor,
-                                                           long a_ld, const eh_desc *__restrict__ descs,
+                                                           long a_ld, const eh_apos *__restrict__ table,
                                                            const eh_fterm *__restrict__ terms, int ne, int t0,
                                                            int t1, int ta0, int n_params, double *gpart,
                                                            double *errpart, const int32_t *cvar) {
   extern __shared__ double g_lds[];
   const int lane = threadIdx.x;
   /* lattice variants: the block (one wavefront) is one 64-entry chunk of one variant */
+  const eh_apos *pos = table;
   if (cvar)
-    descs += (long)cvar[blockIdx.x] * ne;
+    pos += (long)cvar[blockIdx.x] * ne;
   for (int q = lane; q < n_params; q += EH_ADJ_BLOCK)
     g_lds[q] = 0;
   __syncthreads();
@@ -4157,8 +4263,11 @@ k_adj_bwd(double *zb, double *lam, long m, const int32_t *arow,
   double err = 0, err_s = 0;
   for (int t = t1 - 1; t >= t0; t--) {
     const long tb = (long)(t - ta0) * n_anchor;
+    int64_t next_off = pos[ne - 1].off;
     for (int e = ne - 1; e >= 0; e--) {
-      const eh_desc &d = descs[e];
+      const eh_apos *q = pos + e;
+      const eh_desc &d = *(const eh_desc *)((const char *)table + next_off);
+      next_off = pos[e > 0 ? e - 1 : ne - 1].off;
       switch (d.type) {
       case EH_T_DRIF:
         eh_adj_drif(z, l, d.length, d.T11);
@@ -4172,40 +4281,20 @@ k_adj_bwd(double *zb, double *lam, long m, const int32_t *arow,
       case EH_T_KQUSE: {
         eh_pgrad g = {0, 0, 0, 0};
         eh_adj_multipole(z, l, d, g);
-        if (d.adj_pk >= 0) {
-          double v = wave_sum(g.k);
-          if (lane == 0)
-            g_lds[d.adj_pk] += v;
-        }
-        if (d.adj_pdx >= 0) {
-          double v = wave_sum(g.dx);
-          if (lane == 0)
-            g_lds[d.adj_pdx] += v;
-        }
-        if (d.adj_pdy >= 0) {
-          double v = wave_sum(g.dy);
-          if (lane == 0)
-            g_lds[d.adj_pdy] += v;
-        }
+        add_slot(g_lds, q->slot[0], g.k);
+        add_slot(g_lds, q->slot[1], g.dx);
+        add_slot(g_lds, q->slot[2], g.dy);
         break;
       }
       case EH_T_CSBEND: {
         eh_pgrad g = {0, 0, 0, 0};
         eh_adj_csbend(z, l, d, terms, g);
-        if (d.adj_pk >= 0) {
-          double v = wave_sum(g.k);
-          if (lane == 0)
-            g_lds[d.adj_pk] += v;
-        }
-        if (d.adj_pfse >= 0) {
-          double v = wave_sum(g.fse);
-          if (lane == 0)
-            g_lds[d.adj_pfse] += v;
-        }
+        add_slot(g_lds, q->slot[0], g.k);
+        add_slot(g_lds, q->slot[3], g.fse);
         break;
       }
       case EH_T_RFCA: {
-        eh_p6 zin = load_anchor(anchors, tb + (e == 0 ? 0 : d.adj_anchor), a_ld, col);
+        eh_p6 zin = load_anchor(anchors, tb + (e == 0 ? 0 : q->anchor), a_ld, col);
         eh_adj_rfca(z, l, zin, d);
         break;
       }
@@ -4275,7 +4364,7 @@ struct eh_adjoint {
   double *d_ckpt = nullptr;    /* (n_ckpt) x 6 x n turn-start states */
   double *d_anchor = nullptr;  /* anchors: all turns x n (store_all) or one segment x survivors */
   size_t anchor_bytes = 0;
-  eh_desc *d_desc = nullptr;
+  char *d_table = nullptr;     /* adj_table: positions, then the distinct descriptors */
   eh_fterm *d_terms = nullptr;
   unsigned long long *d_cnt = nullptr;
   std::vector<double> z_final; /* 6 x n */
@@ -4296,7 +4385,7 @@ struct eh_adjoint {
 };
 
 static void adj_release(eh_adjoint *a) {
-  void *ptrs[] = {a->d_z, a->d_alive, a->d_ckpt, a->d_anchor, a->d_desc, a->d_terms, a->d_cnt, a->d_cvar};
+  void *ptrs[] = {a->d_z, a->d_alive, a->d_ckpt, a->d_anchor, a->d_table, a->d_terms, a->d_cnt, a->d_cvar};
   for (void *p : ptrs)
     if (p)
       (void)hipFree(p);
@@ -4304,7 +4393,7 @@ static void adj_release(eh_adjoint *a) {
   a->d_alive = nullptr;
   a->d_ckpt = nullptr;
   a->d_anchor = nullptr;
-  a->d_desc = nullptr;
+  a->d_table = nullptr;
   a->d_terms = nullptr;
   a->d_cnt = nullptr;
   a->d_cvar = nullptr;
@@ -4410,6 +4499,7 @@ static long adj_bend_params(eh_desc &d, const EH_CSBEND *cb, std::vector<eh_fter
     }
   }
   d.adj_fse1 = 1 / den;
+  d.adj_per_k1 = b[1] != 0 ? bk[1] / b[1] : 0.0;
   return EH_OK;
 }
 
@@ -4557,7 +4647,8 @@ static long adj_forward_rows(eh_adjoint *a, const std::vector<double> &h, const 
   HIPCHK(hipMalloc(&a->d_z, sizeof(double) * 6 * n));
   HIPCHK(hipMalloc(&a->d_alive, sizeof(int32_t) * n));
   HIPCHK(hipMalloc(&a->d_cnt, sizeof(unsigned long long) * 4));
-  HIPCHK(hipMalloc(&a->d_desc, sizeof(eh_desc) * a->hd.size()));
+  const std::vector<char> table = adj_table(a->hd, a->pool);
+  HIPCHK(hipMalloc(&a->d_table, table.size()));
   HIPCHK(hipMalloc(&a->d_terms, sizeof(eh_fterm) * (a->pool.size() + 1)));
   if (!a->cvar.empty()) {
     HIPCHK(hipMalloc(&a->d_cvar, sizeof(int32_t) * a->cvar.size()));
@@ -4569,7 +4660,7 @@ static long adj_forward_rows(eh_adjoint *a, const std::vector<double> &h, const 
   } else {
     HIPCHK(hipMalloc(&a->d_ckpt, sizeof(double) * 6 * (size_t)n * n_ckpt));
   }
-  HIPCHK(hipMemcpy(a->d_desc, a->hd.data(), sizeof(eh_desc) * a->hd.size(), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(a->d_table, table.data(), table.size(), hipMemcpyHostToDevice));
   if (!a->pool.empty())
     HIPCHK(hipMemcpy(a->d_terms, a->pool.data(), sizeof(eh_fterm) * a->pool.size(), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(a->d_z, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice));
@@ -4586,7 +4677,7 @@ static long adj_forward_rows(eh_adjoint *a, const std::vector<double> &h, const 
       HIPCHK(hipMemcpyAsync(a->d_ckpt + (size_t)k * 6 * n, a->d_z, sizeof(double) * 6 * n, hipMemcpyDeviceToDevice,
                             a->stream));
     hipLaunchKernelGGL(k_adj_fwd, dim3(grid_for(n)), dim3(EH_BLOCK), 0, a->stream, a->d_z, n, a->d_alive, n,
-                       a->d_desc, a->d_terms, (int)ne, t0, t1, anc, n_anchor, n, a->d_cnt, a->d_cvar);
+                       (const eh_apos *)a->d_table, a->d_terms, (int)ne, t0, t1, anc, n_anchor, n, a->d_cnt, a->d_cvar);
     HIPCHK(hipGetLastError());
   }
   long r = adj_timed(a, &a->fwd_ms);
@@ -4870,7 +4961,8 @@ extern "C" long eh_adjoint_backward(eh_adjoint *a, const double *grad_final, dou
           hipLaunchKernelGGL(k_adj_gather, dim3(grid_for(m)), dim3(EH_BLOCK), 0, a->stream,
                              a->d_ckpt + (size_t)k * 6 * n, n, d_surv, m, ztmp);
           hipLaunchKernelGGL(k_adj_fwd, dim3(grid_for(m)), dim3(EH_BLOCK), 0, a->stream, ztmp, m, al1, m,
-                             a->d_desc, a->d_terms, (int)ne, t0, t1, d_seg, a->n_anchor, m, a->d_cnt + 1,
+                             (const eh_apos *)a->d_table, a->d_terms, (int)ne, t0, t1, d_seg, a->n_anchor, m,
+                             a->d_cnt + 1,
                              d_cvar_b);
           e1 = hipGetLastError();
         }
@@ -4892,7 +4984,8 @@ extern "C" long eh_adjoint_backward(eh_adjoint *a, const double *grad_final, dou
       }
       HIPCHK(hipEventRecord(a->ev0, a->stream));
       hipLaunchKernelGGL(k_adj_bwd, dim3((unsigned)nb), dim3(EH_ADJ_BLOCK), lds, a->stream, d_zb, d_lam, m, arow, anc,
-                         a->n_anchor, a_ld, a->d_desc, a->d_terms, (int)ne, t0, t1, ta0, np, d_gpart, d_err,
+                         a->n_anchor, a_ld, (const eh_apos *)a->d_table, a->d_terms, (int)ne, t0, t1, ta0, np, d_gpart,
+                         d_err,
                          d_cvar_b);
       hipError_t e2 = hipGetLastError();
       if (e2 != hipSuccess) {
