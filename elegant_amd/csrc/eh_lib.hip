@@ -1257,12 +1257,14 @@ extern "C" long eh_beam_upload(eh_beam *b, double **coord, long n_part) {
 /* ------------------------------------------------------------------------- */
 /* kernels */
 #define EH_BLOCK 256
-/* Occupancy target for the tracking kernels: six wavefronts per SIMD caps
- * them at 80 VGPRs (512 / 6, in granules of 8).  The compiler's own choice
- * (~90 VGPRs, five wavefronts) leaves the FP64 pipe idle while wavefronts wait
- * on their loads and dependent FP64 chains; the few registers it then spills
- * cost less than the sixth wavefront gains (measured on the MBA ring). */
-#define EH_TRACK_WAVES __attribute__((amdgpu_waves_per_eu(6)))
+/* Occupancy target for the tracking kernels: five wavefronts per SIMD, 96 VGPRs.
+ * The regular integrators are bound by instruction issue, which four or five
+ * wavefronts fill; a sixth only costs spills around them.  Kernel time in ms at 3,
+ * 4, 5, 6 and 8 wavefronts: MBA ring, 2 turns, 1e6 particles 149.6, 148.7, 147.4,
+ * 147.6, 160.5; 30401 particles (one wavefront per SIMD or none) 17.7, 17.1, 17.4,
+ * 17.5, 23.0; with radiation, 5e4 particles, 1 turn 11.7, 11.9, 11.7, 13.2, 17.4;
+ * FODO ring, 1e4 particles, 40 turns 11.2, 11.2, 11.2, 12.3, 14.6. */
+#define EH_TRACK_WAVES __attribute__((amdgpu_waves_per_eu(5)))
 
 __device__ __forceinline__ eh_p6 load_p(const eh_soa a, long i) {
   eh_p6 p;

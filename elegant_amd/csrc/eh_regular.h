@@ -56,10 +56,13 @@
 #ifndef EH_REGULAR_H
 #define EH_REGULAR_H
 
-/* limits of the regular path: 1 + delta, canonical momenta (about the slopes; a
- * bend's QX swings by its sub-step angles on the design orbit already), and the
+/* limits of the regular path: 1 + delta; canonical momenta, about the slopes (a
+ * bend's QX swings by its sub-step angles on the design orbit already); and the
  * smallest non-zero momentum, whose quotients are far from underflow.  With them
- * the series argument below is < 2^-11 and |sin phi| < 2^-4. */
+ * |sin phi| < 2^-4 and the series argument below is < 2^-11 (< 2^-7 with WIDE).
+ * Comparisons are or-ed into one mask (keeping running maxima and minima instead
+ * takes fewer scalar instructions, but v_max_f64 and v_min_f64 cost more than
+ * v_cmp: 1e6 particles 4 % slower). */
 #define EH_REG_B1_MIN 0.875
 #define EH_REG_B1_MAX 1.25
 #define EH_REG_QMAX 0.0117
@@ -117,10 +120,54 @@ EH_HD bool eh_reg_next_recip(double b, double &rh) {
   return eh_fabs(e) < 0x1p-18;
 }
 
+/* The coefficients of the short series, opaque to the compiler on the GPU so that
+ * it keeps them in scalar registers across a bend: known constants it rebuilds at
+ * every use, two s_mov each, which a wavefront alone on its SIMD pays in full (30
+ * of the 200 instructions of a sub-step). */
+struct eh_reg_series {
+  double s1, s2, s3, s4, s5, c2, c3, c4, c5, c6, a1, a2, a3, a4;
+};
+
+EH_HD double eh_reg_keep(double c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __asm__ volatile("" : "+s"(c));
+#endif
+  return c;
+}
+
+EH_HD eh_reg_series eh_reg_series_load() {
+  return {eh_reg_keep(EH_SIN_1),  eh_reg_keep(EH_SIN_2),  eh_reg_keep(EH_SIN_3),  eh_reg_keep(EH_SIN_4),
+          eh_reg_keep(EH_SIN_5),  eh_reg_keep(EH_COS_2),  eh_reg_keep(EH_COS_3),  eh_reg_keep(EH_COS_4),
+          eh_reg_keep(EH_COS_5),  eh_reg_keep(EH_COS_6),  eh_reg_keep(EH_ASIN_1), eh_reg_keep(EH_ASIN_2),
+          eh_reg_keep(EH_ASIN_3), eh_reg_keep(EH_ASIN_4)};
+}
+
+/* eh_sin_poly, and eh_cos_poly with the exact products by 1/2 inside fma */
+EH_HD double eh_reg_sin(double r, const eh_reg_series &k) {
+  const double z = r * r;
+  double q = eh_horner(z, k.s5, k.s4);
+  q = eh_horner(z, q, k.s3);
+  q = eh_horner(z, q, k.s2);
+  q = eh_horner(z, q, k.s1);
+  return eh_fma(r * z, q, r);
+}
+
+EH_HD double eh_reg_cos(double r, const eh_reg_series &k) {
+  const double z = r * r;
+  double p = eh_horner(z, k.c6, k.c5);
+  p = eh_horner(z, p, k.c4);
+  p = eh_horner(z, p, k.c3);
+  p = eh_horner(z, p, k.c2);
+  const double zl = eh_fma(r, r, -z);
+  const double w = eh_fma(-0.5, z, 1.0);
+  const double t = eh_fma(-0.5, z, 1.0 - w);
+  return w + eh_fma(z * z, p, eh_fma(-0.5, zl, t));
+}
+
 /* eh_asin below 2^-4: the two short series of eh_asin_small */
-EH_HD double eh_reg_asin(double x) {
+EH_HD double eh_reg_asin(double x, const eh_reg_series &k) {
   const double z = x * x;
-  double q = EH_ASIN_4;
+  double q = k.a4;
   const bool longer = !(eh_fabs(x) < 0x1p-8);
 #if defined(__HIP_DEVICE_COMPILE__)
   if (__ballot(longer))
@@ -134,9 +181,9 @@ EH_HD double eh_reg_asin(double x) {
     p = eh_horner(z, p, EH_ASIN_4);
     q = longer ? p : q;
   }
-  q = eh_horner(z, q, EH_ASIN_3);
-  q = eh_horner(z, q, EH_ASIN_2);
-  q = eh_horner(z, q, EH_ASIN_1);
+  q = eh_horner(z, q, k.a3);
+  q = eh_horner(z, q, k.a2);
+  q = eh_horner(z, q, k.a1);
   return eh_fma(x * z, q, x);
 }
 
@@ -234,6 +281,8 @@ EH_HD bool eh_mult_regular(const eh_desc &d, int pi, double &x_, double &xp_, do
     qy = eh_reg_div(b1 * yp_, w, yw);
   }
   eh_reg_slopes v = eh_reg_m2s(qx, qy, b1s, rh, rh2);
+  /* a particle in the mid-plane stays there, with qy = 0 */
+  const bool midplane = (qy == 0) & (y == 0) & !steering;
   const int nsl = d.reg_nsl, nsub = d.reg_nsub;
   for (int ik = 0; ik < nsl; ik++) {
     bad |= !((eh_fabs(x + mdx) <= apx) & (eh_fabs(y + mdy) <= apy));
@@ -271,7 +320,7 @@ EH_HD bool eh_mult_regular(const eh_desc &d, int pi, double &x_, double &xp_, do
         }
       }
       const double ax = eh_fabs(qx), ay = eh_fabs(qy);
-      bad |= !((ax <= EH_REG_QMAX) & (ay <= EH_REG_QMAX) & eh_reg_sized(ax) & eh_reg_sized(ay));
+      bad |= !((ax <= EH_REG_QMAX) & (ay <= EH_REG_QMAX) & eh_reg_sized(ax) & ((ay >= EH_REG_QMIN) | midplane));
       if constexpr (RAD) {
         /* the energy loss, as the general integrator forms it; squares hide the
          * signs of zeros and anything near underflow */
@@ -362,29 +411,27 @@ EH_HD bool eh_csb_regular(const eh_desc &d, int pi, const eh_fterm *__restrict__
     const double q2 = QY * QY;
     eh_reg_root(b1s - q2, q2 * rh2, rh, f, y);
   }
+  const eh_reg_series ks = eh_reg_series_load();
   const int nsl = d.reg_nsl, nsub = d.reg_nsub;
+  /* A momentum that stays far above underflow has lost nothing to a tiny, inexact
+   * kick.  QY may be zero throughout: always without field terms, in the mid-plane
+   * with them. */
+  const bool midplane = (QY == 0) & (FIELD == 1 || Y == 0);
   for (int i = 0; i < nsl; i++) {
     bad |= !((eh_fabs(X) <= apx) & (eh_fabs(Y) <= apy) & (eh_fabs(QX) <= EH_REG_QXMAX) &
              (eh_fabs(QX) >= EH_REG_QMIN));
-#if defined(__HIP_DEVICE_COMPILE__)
-    if (__ballot(!bad) == 0)
-      break;
-#else
-    if (bad)
-      break;
-#endif
     for (int j = 0; j < nsub; j++) {
       const double sin_phi = eh_reg_div(QX, f, y);
-      const double phi = eh_reg_asin(sin_phi);
+      const double phi = eh_reg_asin(sin_phi, ks);
       double th = j == 1 || j == 2 ? h1 : h0;
       if (nsub == 8)
         th = d.csb_dshr[j];
       const double ang = th + phi;
       bad |= !(eh_fabs(ang) < 0x1p-4); /* the short series of eh_sincos */
-      const double sine = eh_sin_poly(ang), cosi = eh_cos_poly(ang);
+      const double sine = eh_reg_sin(ang, ks), cosi = eh_reg_cos(ang, ks);
       const double yc = eh_reg_recip1(cosi);
       const double tang = eh_reg_div(sine, cosi, yc);
-      const double cos_phi = eh_cos_poly(phi);
+      const double cos_phi = eh_reg_cos(phi, ks);
       QX = f * sine;
       const double tphi = eh_reg_div(sin_phi, cos_phi, eh_reg_recip1(cos_phi));
       const double factor = eh_reg_div((rho0 + X) * cos_phi, f, y) * (tang - tphi);
@@ -403,14 +450,10 @@ EH_HD bool eh_csb_regular(const eh_desc &d, int pi, const eh_fterm *__restrict__
         eh_grad_eval(gf, X, Y, Fx, Fy);
       if constexpr (FIELD == 3)
         eh_csb_fields(d, terms, X, Y, Fx, Fy);
-      const double ny = u * Fx;
       QX -= eh_reg_div(u * Fy, rho_a, rah);
-      QY += eh_reg_div(ny, rho_a, rah);
-      /* a momentum far above underflow has lost nothing to an inexact tiny
-       * kick; a particle in the mid-plane keeps QY = 0 exactly */
+      QY += eh_reg_div(u * Fx, rho_a, rah);
       const double ax = eh_fabs(QX), ay = eh_fabs(QY);
-      bad |= !((ax <= EH_REG_QXMAX) & (ay <= EH_REG_QMAX) & (ax >= EH_REG_QMIN) &
-               ((ay >= EH_REG_QMIN) | ((QY == 0) & (ny == 0))));
+      bad |= !((ax <= EH_REG_QXMAX) & (ay <= EH_REG_QMAX) & (ax >= EH_REG_QMIN) & ((ay >= EH_REG_QMIN) | midplane));
       if constexpr (RAD) {
         /* the energy loss of the sub-step as the general integrator forms it; its
          * path factor (h^2 + x'^2 + y'^2)^1/2, h = 1 + X / rho0, is (1 + delta) h / f
