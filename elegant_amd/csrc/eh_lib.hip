@@ -1547,6 +1547,46 @@ __global__ void __launch_bounds__(EH_BLOCK) EH_TRACK_WAVES k_fused(eh_soa a, lon
   wave_store(p, in, alive, row0, lpass, levent, b, 0, &cnt[0], g, &cnt[1]);
 }
 
+/* element by element: position ie of the line with the sweeps that follow it, in
+ * place, over the n particles of the last compaction.  A particle lost by an
+ * earlier launch keeps its mark and is left alone; one lost here is marked with
+ * the pass and the event of the stage that lost it (event, +1 MAXAMP, +2 NaN).
+ * cnt[2] counts the losses, cnt[3] the particle-element units.  One launch instead
+ * of a routine and one or two sweeps with a host visit after each: a launch of 1e4
+ * particles through a drift is bound by dispatch, about 5 us, where the host visit
+ * (constants up, counter cleared, two events, counter down) took 30 (FODO ring, 2
+ * turns: 605 launches in 22.5 ms before, 203 in 1.5 now). */
+template <bool RAD>
+__global__ void __launch_bounds__(EH_BLOCK) EH_TRACK_WAVES k_step(eh_soa a, long n, const eh_pos *__restrict__ pos,
+                                                    const eh_fterm *__restrict__ terms, int ie, int pass,
+                                                    int32_t event, unsigned long long *cnt) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const bool alive = i < n && a.levent[i] < 0;
+  const unsigned long long live = __ballot(alive);
+  if (live == 0)
+    return;
+  const eh_pos *q = pos + ie;
+  const eh_desc *d = (const eh_desc *)((const char *)pos + q->off);
+  bool lost = false;
+  if (alive) {
+    eh_p6 p = load_p(a, i);
+    const int st = eh_apply_element_t<RAD>(p, *d, pass, terms, q->z);
+    store_p(a, i, p);
+    if (st >= 0) {
+      lost = true;
+      a.lpass[i] = pass | ((st & EH_STAGE_INHERIT) ? EH_LPASS_INHERIT : 0);
+      a.levent[i] = event + (st & 3);
+    }
+  }
+  const unsigned long long gone = __ballot(lost);
+  if (__lane_id() == __ffsll((unsigned long long)live) - 1) {
+    if (gone)
+      atomicAdd(&cnt[2], (unsigned long long)__popcll(gone));
+    if (d->counted)
+      atomicAdd(&cnt[3], (unsigned long long)__popcll(live));
+  }
+}
+
 /* ------------------------------------------------------------------------- */
 /* batched lattice variants.  Variant v owns the particle region
  * [region_off[v], region_off[v] + capacity_v) (64-aligned), its alive particles at
@@ -2769,8 +2809,58 @@ static long launch_fused(eh_beam *b, long ne, int p0, int e0, int p1, int e1, do
   return b->n_alive;
 }
 
+/* one pass from element e0 to e1 (exclusive), element by element in place
+ * (k_step), with a host visit at the end only: survivors are compacted there */
+static long launch_steps(eh_beam *b, const EH_ELEMENT_LIST *bl, long ne, int pass, long e0, long e1, int32_t base,
+                         bool rad, double *effort) {
+  const long n = b->n_alive;
+  long count = 0;
+  if (n == 0)
+    return 0;
+  unsigned long long zero[2] = {0, 0};
+  HIPCHK(hipMemcpyAsync(b->d_cnt + 2, zero, sizeof zero, hipMemcpyHostToDevice, b->stream));
+  long r = timed_begin(b);
+  if (r < 0)
+    return r;
+  for (long ie = e0; ie < e1; ie++) {
+    if (bl[ie].type == EH_T_MARK)
+      continue;
+    if (rad)
+      hipLaunchKernelGGL(k_step<true>, dim3(grid_for(n)), dim3(EH_BLOCK), 0, b->stream, b->buf[b->cur], n,
+                         (const eh_pos *)b->d_fused, b->d_terms, (int)ie, pass, base + (int32_t)ie * 3, b->d_cnt);
+    else
+      hipLaunchKernelGGL(k_step<false>, dim3(grid_for(n)), dim3(EH_BLOCK), 0, b->stream, b->buf[b->cur], n,
+                         (const eh_pos *)b->d_fused, b->d_terms, (int)ie, pass, base + (int32_t)ie * 3, b->d_cnt);
+    HIPCHK(hipGetLastError());
+    count++;
+  }
+  if (!count)
+    return n;
+  r = timed_end(b);
+  if (r < 0)
+    return r;
+  b->launches += count - 1;
+  unsigned long long out[2];
+  HIPCHK(hipMemcpy(out, b->d_cnt + 2, sizeof out, hipMemcpyDeviceToHost));
+  *effort += (double)out[1];
+  b->main_ms += b->last_ms;
+  b->main_launches += count;
+  b->main_units += (double)out[1];
+  const long lost0 = b->n_lost;
+  r = compact(b, (long)out[0]);
+  if (r < 0)
+    return r;
+  if (b->n_lost - lost0 != (long)out[0] || b->n_alive != n - (long)out[0])
+    return fail(EH_ERR_STATE, "compaction count mismatch: %ld in, %llu marked lost, %ld kept, %ld buried", n, out[0],
+                b->n_alive, b->n_lost - lost0);
+  return b->n_alive;
+}
+
+/* steps: element by element (EH_MODE_PLAIN), for lines whose elements need
+ * nothing of the beam between them but a cavity's phase on pass 0; the others go
+ * through track_plain */
 static long track_fused(eh_beam *b, EH_ELEMENT_LIST *bl, long ne, long n_passes, double *Pc, int tpl,
-                        double *effort) {
+                        double *effort, bool steps = false) {
   if (tpl < 1)
     tpl = 1;
   long r;
@@ -2845,6 +2935,8 @@ static long track_fused(eh_beam *b, EH_ELEMENT_LIST *bl, long ne, long n_passes,
     }
     dynamic = dynamic || stop_before[ie] || stop_after[ie];
   }
+  if (steps && (dynamic || two_phase))
+    return track_plain(b, bl, ne, n_passes, Pc, effort);
   std::vector<double> Pdyn;
   if (dynamic) {
     Pdyn = Pe0;
@@ -2974,6 +3066,41 @@ static long track_fused(eh_beam *b, EH_ELEMENT_LIST *bl, long ne, long n_passes,
     }
     return upload_fused_descs(b, hd, pool);
   };
+  if (steps) {
+    const long span = ne * 3 + 3;
+    for (int pass = 0; pass < n_passes && b->n_alive > 0; pass++) {
+      if ((long)b->event + span >= 2147483647L)
+        return fail(EH_ERR_STATE, "loss event counter overflow");
+      const int32_t base = b->event;
+      b->event += (int32_t)span;
+      const long lost0 = b->n_lost;
+      if (tab)
+        b->evlog.push_back({base, (int32_t)span, pass, (int32_t)ne, tab, nullptr});
+      b->pass = pass;
+      long e0 = 0;
+      for (long ie = 0; ie <= ne; ie++) {
+        if (ie < ne && !(pass == 0 && pend[ie]))
+          continue;
+        r = launch_steps(b, bl, ne, pass, e0, ie, base, rad, effort);
+        if (r < 0)
+          return r;
+        e0 = ie;
+        if (b->n_alive == 0)
+          break; /* no particle reaches the cavity: the reference takes no fiducial */
+        if (ie < ne) {
+          r = resolve_pending(ie);
+          if (r < 0)
+            return r;
+        }
+      }
+      if (tab && b->n_lost == lost0)
+        b->evlog.pop_back(); /* nothing to settle */
+    }
+    if (n_passes > 0)
+      *Pc = P_end;
+    b->pass = n_passes > 0 ? n_passes - 1 : 0;
+    return b->n_alive;
+  }
   int p = 0, e = 0;
   if (dynamic) {
     /* the reference momentum P at the position (p, e); the momentum each
@@ -3160,7 +3287,7 @@ extern "C" long eh_do_tracking(eh_beam *b, EH_ELEMENT_LIST *beamline, long n_ele
   long l0 = b->launches, ml0 = b->main_launches;
   long r;
   if (mode == EH_MODE_PLAIN)
-    r = track_plain(b, beamline, n_elements, n_passes, P_central, &effort);
+    r = track_fused(b, beamline, n_elements, n_passes, P_central, 1, &effort, true);
   else if (mode == EH_MODE_FUSED)
     r = track_fused(b, beamline, n_elements, n_passes, P_central, turns_per_launch, &effort);
   else

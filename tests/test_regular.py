@@ -149,10 +149,11 @@ def test_who_is_regular(name):
 def test_gpu_matches_oracle(ehlib, name):
     rows = np.concatenate([particles()] * 3)
     rows[:, 6] = np.arange(1, len(rows) + 1)
-    beam = tracking.Beam(rows)
-    n, _, _ = tracking.track(beam, line(name), 2, Po, mode="fused", turns_per_launch=2)
-    got = beam.download()
-    beam.free()
     ref, nref, _, _ = oracle.do_tracking(rows, line(name), 2, Po)
-    assert n == nref
-    check(got, ref, name)
+    for mode in ("fused", "plain"):  # registers through the line; in place, element by element
+        beam = tracking.Beam(rows)
+        n, st, _ = tracking.track(beam, line(name), 2, Po, mode=mode, turns_per_launch=2)
+        got = beam.download()
+        beam.free()
+        assert n == nref
+        check(got, ref, name + " " + mode)
