@@ -1090,7 +1090,12 @@ struct eh_beam {
   eh_fterm *d_terms = nullptr; /* CSBEND field-term pool */
   long terms_cap = 0;
   EH_VMATRIX *d_mat = nullptr; /* transport map of eh_track_particles */
-  std::vector<double> cols; /* columns 6..9 of each uploaded row, by row0 */
+  /* columns 6..9 of each uploaded row, by row0: on the device, so that rows are
+   * taken apart and put together there; on the host for a beam so large that they
+   * do not fit (d_cols is null then) */
+  double *d_cols = nullptr;
+  std::vector<double> cols;
+  size_t region = 0; /* bytes of one of the three regions of mem */
   long pass = 0;
   int32_t event = 0;
   hipStream_t stream = nullptr;
@@ -1169,11 +1174,16 @@ extern "C" eh_beam *eh_beam_create(long n_capacity) {
     n_capacity = 1;
   eh_beam *b = new eh_beam();
   size_t per = soa_bytes(n_capacity);
-  per = (per + 255) & ~(size_t)255;
+  per = std::max((per + 255) & ~(size_t)255, (size_t)4096); /* the least row_scratch divides up */
   if (hipMalloc(&b->mem, 3 * per) != hipSuccess) {
     fail(EH_ERR_NOMEM, "hipMalloc of %zu bytes failed", 3 * per);
     delete b;
     return nullptr;
+  }
+  b->region = per;
+  if (hipMalloc(&b->d_cols, sizeof(double) * 4 * n_capacity) != hipSuccess) {
+    (void)hipGetLastError();
+    b->d_cols = nullptr;
   }
   soa_carve(&b->buf[0], (char *)b->mem, n_capacity);
   soa_carve(&b->buf[1], (char *)b->mem + per, n_capacity);
@@ -1184,6 +1194,7 @@ extern "C" eh_beam *eh_beam_create(long n_capacity) {
       hipEventCreate(&b->ev1) != hipSuccess) {
     fail(EH_ERR_HIP, "beam setup failed");
     (void)hipFree(b->mem);
+    (void)hipFree(b->d_cols);
     delete b;
     return nullptr;
   }
@@ -1196,6 +1207,8 @@ extern "C" void eh_beam_free(eh_beam *b) {
     return;
   if (b->stream)
     (void)hipStreamSynchronize(b->stream);
+  if (b->d_cols)
+    (void)hipFree(b->d_cols);
   (void)hipFree(b->mem);
   (void)hipFree(b->d_cnt);
   if (b->d_mat)
@@ -1222,28 +1235,148 @@ extern "C" void eh_beam_set_pass(eh_beam *b, long pass) {
     b->pass = pass;
 }
 
-extern "C" long eh_beam_upload(eh_beam *b, double **coord, long n_part) {
-  if (!b || !coord || n_part < 0 || n_part > b->n_total)
-    return fail(EH_ERR_ARG, "eh_beam_upload: bad arguments (n_part=%ld, capacity=%ld)", n_part,
-                b ? b->n_total : 0L);
-  std::vector<double> h(6 * (size_t)n_part);
-  std::vector<int32_t> r(n_part), m1(n_part, -1), z(n_part, 0);
-  b->cols.assign(4 * (size_t)n_part, 0.0);
-  for (long i = 0; i < n_part; i++) {
-    for (int k = 0; k < 6; k++)
-      h[k * (size_t)n_part + i] = coord[i][k];
+/* rows of EH_NPROP doubles to columns and back.  A row is 80 consecutive bytes,
+ * which one thread reads or writes: 64 of them cover 40 whole 128-byte lines, so
+ * the device side costs the copy of the rows at HBM rate and the call the transfer
+ * of the rows over PCIe, in chunks through the region of mem that holds no
+ * particles.  On the host, one loop took the 1e6 rows apart (23 ms) and another
+ * put them together (23 ms). */
+__global__ void k_unpack(const double *__restrict__ rows, long r0, long n, eh_soa a, double *__restrict__ cols) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n)
+    return;
+  const double *c = rows + i * EH_NPROP;
+  const long r = r0 + i;
+  a.x[r] = c[0];
+  a.xp[r] = c[1];
+  a.y[r] = c[2];
+  a.yp[r] = c[3];
+  a.s[r] = c[4];
+  a.dp[r] = c[5];
+  a.row0[r] = (int32_t)r;
+  a.lpass[r] = 0;
+  a.levent[r] = -1;
+  if (cols)
     for (int k = 0; k < 4; k++)
-      b->cols[4 * (size_t)i + k] = coord[i][6 + k];
-    r[i] = (int32_t)i;
+      cols[4 * r + k] = c[6 + k];
+}
+
+/* where each identity is: slot k of the survivors, or -1 - k of the graveyard */
+__global__ void k_slots(const int32_t *__restrict__ row0, long n, bool grave, long N, int32_t *__restrict__ slot_of) {
+  const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n)
+    return;
+  const int32_t id = row0[k];
+  if (id >= 0 && id < N)
+    slot_of[id] = grave ? -1 - (int32_t)k : (int32_t)k;
+}
+
+#define EH_NO_SLOT INT32_MIN
+
+__global__ void k_fill_slots(int32_t *p, long n) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n)
+    p[i] = EH_NO_SLOT;
+}
+
+/* rows [r0, r0 + n) of the reference's arrangement (identity slot_at[r], or r
+ * where nothing was lost); a missing identity is counted in cnt[4] */
+__global__ void k_pack(eh_soa a, eh_soa g, const double *__restrict__ cols, const int32_t *__restrict__ slot_of,
+                       const int32_t *__restrict__ slot_at, long r0, long n, double *__restrict__ rows,
+                       unsigned long long *cnt) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n)
+    return;
+  const long id = slot_at ? slot_at[r0 + i] : r0 + i;
+  const int32_t s = slot_of[id];
+  if (s == EH_NO_SLOT) {
+    atomicAdd(&cnt[4], 1ull);
+    return;
   }
-  eh_soa &a = b->buf[0];
+  double *c = rows + i * EH_NPROP;
+  const eh_soa &from = s >= 0 ? a : g;
+  const long k = s >= 0 ? s : -1 - (long)s;
+  c[0] = from.x[k];
+  c[1] = from.xp[k];
+  c[2] = from.y[k];
+  c[3] = from.yp[k];
+  c[4] = from.s[k];
+  c[5] = from.dp[k];
+  if (cols)
+    for (int q = 0; q < 4; q++)
+      c[6 + q] = cols[4 * id + q];
+}
+
+/* arrival times (s + sOffset) / (c beta) of the survivors, rows [0, n) of the
+ * reference's arrangement; a row whose particle is not alive is counted in cnt[4] */
+__global__ void k_arrival(eh_soa a, const int32_t *__restrict__ slot_of, const int32_t *__restrict__ slot_at, long n,
+                          double sOffset, double p0, double *__restrict__ out, unsigned long long *cnt) {
+  const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= n)
+    return;
+  const int32_t k = slot_of[slot_at ? slot_at[r] : r];
+  if (k < 0) {
+    atomicAdd(&cnt[4], 1ull);
+    return;
+  }
+  double p = p0;
+  p *= 1 + a.dp[k];
+  const double beta = p / eh_sqrt(p * p + 1);
+  out[r] = (a.s[k] + sOffset) / (2.99792458e8 * beta);
+}
+
+static unsigned grid_of(long n) { return (unsigned)((n + 255) / 256); }
+
+/* the region without particles as two maps of N identities and a buffer */
+struct eh_row_scratch {
+  int32_t *slot_of, *slot_at;
+  char *buf;
+  long bytes;
+};
+
+static eh_row_scratch row_scratch(eh_beam *b, long N) {
+  eh_row_scratch s;
+  char *base = (char *)b->mem + (size_t)(1 - b->cur) * b->region;
+  s.slot_of = (int32_t *)base;
+  s.slot_at = s.slot_of + N;
+  const size_t used = ((size_t)N * 8 + 255) & ~(size_t)255;
+  s.buf = base + used;
+  s.bytes = (long)(b->region - used);
+  return s;
+}
+
+/* rows per chunk: enough for the transfer's rate, small enough to overlap */
+#define EH_CHUNK_ROWS 262144l
+
+/* n_part rows, consecutive (flat) or by pointer */
+static long upload_rows(eh_beam *b, const double *flat, double **coord, long n_part) {
   b->cur = 0;
-  double *dst[6] = {a.x, a.xp, a.y, a.yp, a.s, a.dp};
-  for (int k = 0; k < 6; k++)
-    HIPCHK(hipMemcpy(dst[k], h.data() + k * (size_t)n_part, sizeof(double) * n_part, hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(a.row0, r.data(), sizeof(int32_t) * n_part, hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(a.levent, m1.data(), sizeof(int32_t) * n_part, hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(a.lpass, z.data(), sizeof(int32_t) * n_part, hipMemcpyHostToDevice));
+  const long chunk = std::min(EH_CHUNK_ROWS, (long)(b->region / (sizeof(double) * EH_NPROP)));
+  char *buf = (char *)b->mem + b->region;
+  std::vector<double> rows;
+  b->cols.clear();
+  if (!b->d_cols)
+    b->cols.resize(4 * (size_t)n_part);
+  for (long r0 = 0; r0 < n_part; r0 += chunk) {
+    const long n = std::min(chunk, n_part - r0);
+    const double *src = flat ? flat + r0 * EH_NPROP : nullptr;
+    if (!src) {
+      rows.resize((size_t)n * EH_NPROP);
+      for (long i = 0; i < n; i++)
+        std::memcpy(&rows[(size_t)i * EH_NPROP], coord[r0 + i], sizeof(double) * EH_NPROP);
+      src = rows.data();
+    }
+    if (!b->d_cols)
+      for (long i = 0; i < n; i++)
+        std::memcpy(&b->cols[4 * (size_t)(r0 + i)], src + i * EH_NPROP + 6, sizeof(double) * 4);
+    HIPCHK(hipMemcpyAsync(buf, src, sizeof(double) * EH_NPROP * n, hipMemcpyHostToDevice, b->stream));
+    hipLaunchKernelGGL(k_unpack, dim3(grid_of(n)), dim3(256), 0, b->stream, (const double *)buf, r0, n, b->buf[0],
+                       b->d_cols);
+    HIPCHK(hipGetLastError());
+    /* the next chunk goes into the same buffer, and the caller's rows are free to
+     * change on return */
+    HIPCHK(hipStreamSynchronize(b->stream));
+  }
   b->n_alive = n_part;
   b->n_lost = 0;
   b->event = 0;
@@ -1252,6 +1385,16 @@ extern "C" long eh_beam_upload(eh_beam *b, double **coord, long n_part) {
   b->kernel_ms = 0;
   b->launches = 0;
   return n_part;
+}
+
+extern "C" long eh_beam_upload(eh_beam *b, double **coord, long n_part) {
+  if (!b || !coord || n_part < 0 || n_part > b->n_total)
+    return fail(EH_ERR_ARG, "eh_beam_upload: bad arguments (n_part=%ld, capacity=%ld)", n_part,
+                b ? b->n_total : 0L);
+  bool flat = true; /* czarray_2d lays the rows out one after the other */
+  for (long i = 1; i < n_part && flat; i++)
+    flat = coord[i] == coord[0] + i * EH_NPROP;
+  return upload_rows(b, flat && n_part > 0 ? coord[0] : nullptr, coord, n_part);
 }
 
 /* ------------------------------------------------------------------------- */
@@ -2140,11 +2283,45 @@ extern "C" long eh_elimit_amplitudes(eh_beam *b, double xmax, double ymax, long 
 static long reference_order(eh_beam *b, std::vector<int32_t> &slot_at_row, std::vector<int32_t> &alive_row0,
                             std::vector<int32_t> &dev_index_alive, std::vector<int32_t> *pred = nullptr,
                             std::vector<int32_t> *order = nullptr);
+static long device_order(eh_beam *b, const eh_row_scratch &s, std::vector<int32_t> &slot_at_row,
+                         std::vector<int32_t> &pred, std::vector<int32_t> &order, std::vector<int32_t> &gidx,
+                         std::vector<int32_t> &gev);
+static long check_missing(eh_beam *b, const char *what);
 static long fiducial_from_beam(eh_beam *b, int mode, double sOffset, double p0, double *tFid) {
   if (mode == EH_FID_FIRST)
     return fail(EH_ERR_ARG, "No available particle for the FID_MODE_FIRST mode in findFiducialTime");
+  long r;
+  if (mode == EH_FID_TMEAN) {
+    /* the arrival times in the reference's row order from the device; their Kahan
+     * sum is a serial chain, which the host runs */
+    const long n = b->n_alive;
+    const eh_row_scratch s = row_scratch(b, n + b->n_lost);
+    std::vector<int32_t> slot_at_row, pred, order, gidx, gev;
+    r = device_order(b, s, slot_at_row, pred, order, gidx, gev);
+    if (r < 0)
+      return r;
+    std::vector<double> t(n);
+    if (n) {
+      hipLaunchKernelGGL(k_arrival, dim3(grid_of(n)), dim3(256), 0, b->stream, b->buf[b->cur], s.slot_of,
+                         b->n_lost ? s.slot_at : nullptr, n, sOffset, p0, (double *)s.buf, b->d_cnt);
+      HIPCHK(hipGetLastError());
+      HIPCHK(hipMemcpyAsync(t.data(), s.buf, sizeof(double) * n, hipMemcpyDeviceToHost, b->stream));
+      r = check_missing(b, "the RF fiducial");
+      if (r < 0)
+        return r;
+    }
+    double tsum = 0, error = 0.0;
+    for (long row = 0; row < n; row++) {
+      double Y = t[row] + error;
+      double sum = tsum + Y;
+      error = Y - (sum - tsum);
+      tsum = sum;
+    }
+    *tFid = n > 0 ? tsum / n : 0.0;
+    return EH_OK;
+  }
   std::vector<int32_t> slot_at_row, alive_row0, idx;
-  long r = reference_order(b, slot_at_row, alive_row0, idx);
+  r = reference_order(b, slot_at_row, alive_row0, idx);
   if (r < 0)
     return r;
   long n = b->n_alive;
@@ -2178,17 +2355,7 @@ static long fiducial_from_beam(eh_beam *b, int mode, double sOffset, double p0, 
     *tFid = t_of(dev[ibest]);
     return EH_OK;
   }
-  double tsum = 0, error = 0.0;
-  long nsum = 0;
-  for (long row = 0; row < n; row++) {
-    double Y = t_of(dev[row]) + error;
-    double sum = tsum + Y;
-    error = Y - (sum - tsum);
-    tsum = sum;
-    nsum++;
-  }
-  *tFid = nsum > 0 ? tsum / nsum : 0.0;
-  return EH_OK;
+  return fail(EH_ERR_ARG, "invalid fiducial mode for RFCA element");
 }
 
 /* do_match_energy (src/do_tracking.c:3376-3549, serial elegant with USE_KAHAN):
@@ -2584,56 +2751,121 @@ static long reference_order(eh_beam *b, std::vector<int32_t> &slot_at_row, std::
   return EH_OK;
 }
 
-extern "C" long eh_beam_download(eh_beam *b, double **coord, long n_part) {
-  if (!b || !coord)
-    return fail(EH_ERR_ARG, "eh_beam_download: null argument");
-  long N = b->n_alive + b->n_lost;
+/* the maps of row_scratch on the device: slot_of always, slot_at if anything was
+ * lost (slot_at_row, pred and order then hold the replay, gidx the graveyard slot
+ * of each lost identity and gev its event).  Clears cnt[4]. */
+static long device_order(eh_beam *b, const eh_row_scratch &s, std::vector<int32_t> &slot_at_row,
+                         std::vector<int32_t> &pred, std::vector<int32_t> &order, std::vector<int32_t> &gidx,
+                         std::vector<int32_t> &gev) {
+  const long na = b->n_alive, nl = b->n_lost, N = na + nl;
+  if (!N)
+    return EH_OK;
+  const unsigned long long zero = 0;
+  HIPCHK(hipMemcpyAsync(b->d_cnt + 4, &zero, sizeof zero, hipMemcpyHostToDevice, b->stream));
+  hipLaunchKernelGGL(k_fill_slots, dim3(grid_of(N)), dim3(256), 0, b->stream, s.slot_of, N);
+  if (na)
+    hipLaunchKernelGGL(k_slots, dim3(grid_of(na)), dim3(256), 0, b->stream, b->buf[b->cur].row0, na, false, N,
+                       s.slot_of);
+  if (nl)
+    hipLaunchKernelGGL(k_slots, dim3(grid_of(nl)), dim3(256), 0, b->stream, b->grave.row0, nl, true, N, s.slot_of);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(b->stream));
+  slot_at_row.clear();
+  if (!nl)
+    return EH_OK;
+  std::vector<int32_t> grow0(nl);
+  gev.resize(nl);
+  gidx.assign(N, -1);
+  HIPCHK(hipMemcpy(grow0.data(), b->grave.row0, sizeof(int32_t) * nl, hipMemcpyDeviceToHost));
+  HIPCHK(hipMemcpy(gev.data(), b->grave.levent, sizeof(int32_t) * nl, hipMemcpyDeviceToHost));
+  std::vector<std::pair<int32_t, int32_t>> lost(nl);
+  for (long k = 0; k < nl; k++) {
+    if (grow0[k] < 0 || grow0[k] >= N)
+      return fail(EH_ERR_STATE, "corrupt particle identity");
+    lost[k] = std::make_pair(gev[k], grow0[k]);
+    gidx[grow0[k]] = (int32_t)k;
+  }
+  replay_order(N, lost, slot_at_row, &pred, &order);
+  HIPCHK(hipMemcpy(s.slot_at, slot_at_row.data(), sizeof(int32_t) * N, hipMemcpyHostToDevice));
+  return EH_OK;
+}
+
+static long check_missing(eh_beam *b, const char *what) {
+  unsigned long long missing = 0;
+  HIPCHK(hipMemcpyAsync(&missing, b->d_cnt + 4, sizeof missing, hipMemcpyDeviceToHost, b->stream));
+  HIPCHK(hipStreamSynchronize(b->stream));
+  if (missing)
+    return fail(EH_ERR_STATE, "%llu particles missing on %s", missing, what);
+  return EH_OK;
+}
+
+/* the reference's arrangement into n_part rows, consecutive (flat) or by pointer */
+static long download_rows(eh_beam *b, double *flat, double **coord, long n_part) {
+  const long na = b->n_alive, nl = b->n_lost, N = na + nl;
   if (n_part != N)
     return fail(EH_ERR_ARG, "eh_beam_download: n_part=%ld but the beam holds %ld particles", n_part, N);
-  std::vector<int32_t> slot_at_row, alive_row0, idx, pred, order;
-  long r = reference_order(b, slot_at_row, alive_row0, idx, &pred, &order);
+  const eh_row_scratch s = row_scratch(b, N);
+  std::vector<int32_t> slot_at_row, pred, order, gidx, gev;
+  long r = device_order(b, s, slot_at_row, pred, order, gidx, gev);
   if (r < 0)
     return r;
-  long na = b->n_alive, nl = b->n_lost;
-  std::vector<double> A(6 * (size_t)na), G(6 * (size_t)nl);
-  std::vector<int32_t> grow0(nl), gpass(nl);
-  const eh_soa &a = b->buf[b->cur], &g = b->grave;
-  const double *as[6] = {a.x, a.xp, a.y, a.yp, a.s, a.dp}, *gs[6] = {g.x, g.xp, g.y, g.yp, g.s, g.dp};
-  for (int k = 0; k < 6; k++) {
-    if (na)
-      HIPCHK(hipMemcpy(A.data() + k * (size_t)na, as[k], sizeof(double) * na, hipMemcpyDeviceToHost));
-    if (nl)
-      HIPCHK(hipMemcpy(G.data() + k * (size_t)nl, gs[k], sizeof(double) * nl, hipMemcpyDeviceToHost));
+  const long chunk = std::min(EH_CHUNK_ROWS, s.bytes / (long)(sizeof(double) * EH_NPROP));
+  std::vector<double> rows;
+  for (long r0 = 0; r0 < N; r0 += chunk) {
+    const long n = std::min(chunk, N - r0);
+    hipLaunchKernelGGL(k_pack, dim3(grid_of(n)), dim3(256), 0, b->stream, b->buf[b->cur], b->grave, b->d_cols,
+                       s.slot_of, nl ? s.slot_at : nullptr, r0, n, (double *)s.buf, b->d_cnt);
+    HIPCHK(hipGetLastError());
+    if (!flat)
+      rows.resize((size_t)n * EH_NPROP);
+    double *dst = flat ? flat + r0 * EH_NPROP : rows.data();
+    HIPCHK(hipMemcpyAsync(dst, s.buf, sizeof(double) * EH_NPROP * n, hipMemcpyDeviceToHost, b->stream));
+    HIPCHK(hipStreamSynchronize(b->stream));
+    for (long i = 0; i < n; i++) {
+      if (!b->d_cols) {
+        const long id = nl ? slot_at_row[r0 + i] : r0 + i;
+        std::memcpy(dst + i * EH_NPROP + 6, &b->cols[4 * (size_t)id], sizeof(double) * 4);
+      } else if (flat)
+        break;
+      if (!flat)
+        std::memcpy(coord[r0 + i], dst + i * EH_NPROP, sizeof(double) * EH_NPROP);
+    }
+  }
+  if (N) {
+    r = check_missing(b, "download");
+    if (r < 0)
+      return r;
   }
   if (nl) {
-    HIPCHK(hipMemcpy(grow0.data(), g.row0, sizeof(int32_t) * nl, hipMemcpyDeviceToHost));
+    /* the lost rows' positions and passes, settled in the reference's order */
+    const eh_soa &g = b->grave;
+    std::vector<double> G(6 * (size_t)nl);
+    std::vector<int32_t> gpass(nl);
+    const double *gs[6] = {nullptr, g.xp, nullptr, g.yp, g.s, nullptr}; /* what settle_losses reads */
+    for (int k = 0; k < 6; k++)
+      if (gs[k])
+        HIPCHK(hipMemcpy(G.data() + k * (size_t)nl, gs[k], sizeof(double) * nl, hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(gpass.data(), g.lpass, sizeof(int32_t) * nl, hipMemcpyDeviceToHost));
-  }
-  std::vector<int32_t> gidx(N, -1), gev(nl);
-  for (long k = 0; k < nl; k++)
-    gidx[grow0[k]] = (int32_t)k;
-  if (nl)
-    HIPCHK(hipMemcpy(gev.data(), g.levent, sizeof(int32_t) * nl, hipMemcpyDeviceToHost));
-  settle_losses(b->evlog, -1, order, pred, gidx, gev, G, nl, gpass);
-  for (long row = 0; row < N; row++) {
-    int32_t id = slot_at_row[row];
-    double *c = coord[row];
-    for (int k = 0; k < 4; k++)
-      c[6 + k] = b->cols[4 * (size_t)id + k];
-    if (idx[id] >= 0) {
-      long k = idx[id];
-      for (int q = 0; q < 6; q++)
-        c[q] = A[q * (size_t)na + k];
-    } else {
-      long k = gidx[id];
+    settle_losses(b->evlog, -1, order, pred, gidx, gev, G, nl, gpass);
+    for (long row = na; row < N; row++) {
+      const long k = gidx[slot_at_row[row]];
       if (k < 0)
-        return fail(EH_ERR_STATE, "particle %d missing on download", id);
-      for (int q = 0; q < 6; q++)
-        c[q] = G[q * (size_t)nl + k];
+        return fail(EH_ERR_STATE, "replay placed a survivor among the lost particles");
+      double *c = flat ? flat + row * EH_NPROP : coord[row];
+      c[4] = G[4 * (size_t)nl + k];
       c[EH_LOSS_PASS_INDEX] = gpass[k];
     }
   }
   return na;
+}
+
+extern "C" long eh_beam_download(eh_beam *b, double **coord, long n_part) {
+  if (!b || !coord)
+    return fail(EH_ERR_ARG, "eh_beam_download: null argument");
+  bool flat = true;
+  for (long i = 1; i < n_part && flat; i++)
+    flat = coord[i] == coord[0] + i * EH_NPROP;
+  return download_rows(b, flat && n_part > 0 ? coord[0] : nullptr, coord, n_part);
 }
 
 extern "C" long eh_beam_row_order(eh_beam *b, int32_t *upload_row, long n_part) {
@@ -3353,21 +3585,15 @@ extern "C" long eh_do_tracking_noalloc(eh_beam *b, EH_ELEMENT_LIST *beamline, lo
 
 /* contiguous AoS variants: rows of EH_NPROP doubles, as czarray_2d lays them out */
 extern "C" long eh_beam_upload_flat(eh_beam *b, const double *flat, long n_part) {
-  if (!flat || n_part < 0)
+  if (!b || !flat || n_part < 0 || n_part > b->n_total)
     return fail(EH_ERR_ARG, "eh_beam_upload_flat: bad arguments");
-  std::vector<double *> rows(n_part > 0 ? n_part : 1);
-  for (long i = 0; i < n_part; i++)
-    rows[i] = const_cast<double *>(flat) + i * EH_NPROP;
-  return eh_beam_upload(b, rows.data(), n_part);
+  return upload_rows(b, flat, nullptr, n_part);
 }
 
 extern "C" long eh_beam_download_flat(eh_beam *b, double *flat, long n_part) {
-  if (!flat || n_part < 0)
+  if (!b || !flat || n_part < 0)
     return fail(EH_ERR_ARG, "eh_beam_download_flat: bad arguments");
-  std::vector<double *> rows(n_part > 0 ? n_part : 1);
-  for (long i = 0; i < n_part; i++)
-    rows[i] = flat + i * EH_NPROP;
-  return eh_beam_download(b, rows.data(), n_part);
+  return download_rows(b, flat, nullptr, n_part);
 }
 
 /* ------------------------------------------------------------------------- */

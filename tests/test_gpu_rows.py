@@ -1,0 +1,62 @@
+"""Rows up and down: taken apart and put together on the device, in chunks of
+262144, with losses moved to the reference's places.  Bit for bit with the oracle."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from elegant_amd import _lib, configs, structs as S, tracking
+from elegant_amd.lattice import Element, Lattice
+from tests.helpers import assert_rows_identical
+
+pytestmark = pytest.mark.gpu
+Po = configs.p_central_from_mev(3000.0)
+
+
+def line():
+    return Lattice([Element("AP", "MAXAMP", X_MAX=0.01, Y_MAX=0.008), Element("D", "DRIF", L=1.0),
+                    Element("Q", "KQUAD", L=0.2, K1=1.0, N_KICKS=4, DX=1e-4), Element("D", "DRIF", L=0.7)])
+
+
+def rows_of(n, spread):
+    rng = np.random.default_rng(n)
+    rows = rng.standard_normal((n, S.NPROP)) * [spread, 1e-3, spread, 1e-3, 1e-3, 1e-3, 1, 1, 1, 1]
+    rows[:, 6] = np.arange(1, n + 1)
+    return rows
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 1000, 262144, 262145, 600001])
+@pytest.mark.parametrize("spread", [1e-4, 6e-3, 1.0])  # none, some, nearly all lost
+def test_rows_round_trip(ehlib, oracle_mod, n, spread):
+    rows = rows_of(n, spread)
+    beam = tracking.Beam(rows)
+    assert_rows_identical(beam.download(), rows, beam.n_alive(), n, "untracked")
+    na, _, _ = tracking.track(beam, line(), 2, Po, mode="fused", turns_per_launch=1)
+    got = beam.download()
+    ref, nref, _, _ = oracle_mod.do_tracking(rows, line(), 2, Po)
+    assert_rows_identical(got, ref, na, nref, "n=%d spread=%g" % (n, spread))
+    order = beam.row_order()
+    assert np.array_equal(rows[order, 6], got[:, 6])
+    beam.free()
+
+
+@pytest.mark.parametrize("n", [5, 262150])
+def test_rows_by_pointer(ehlib, oracle_mod, n):
+    """rows scattered in memory, as a caller may hand them over"""
+    rows = rows_of(n, 6e-3)
+    place = np.random.default_rng(1).permutation(n)
+    store = np.zeros((n, S.NPROP + 3))
+    store[place, :S.NPROP] = rows
+    ptr = (store.ctypes.data + place.astype(np.uint64) * np.uint64(store.strides[0])).astype(np.uint64)
+    L = tracking.lib()
+    L.eh_beam_upload.argtypes = [C.c_void_p, C.c_void_p, C.c_long]
+    L.eh_beam_download.argtypes = [C.c_void_p, C.c_void_p, C.c_long]
+    beam = tracking.Beam(rows_of(n, 1e-4), capacity=n + 17)
+    _lib.check(L.eh_beam_upload(beam.handle, ptr.ctypes.data, n))
+    na, _, _ = tracking.track(beam, line(), 1, Po, mode="plain")
+    store[:] = -7.0
+    _lib.check(L.eh_beam_download(beam.handle, ptr.ctypes.data, n))
+    ref, nref, _, _ = oracle_mod.do_tracking(rows, line(), 1, Po)
+    assert_rows_identical(store[place, :S.NPROP], ref, na, nref, "by pointer")
+    assert (store[:, S.NPROP:] == -7.0).all()
+    beam.free()
