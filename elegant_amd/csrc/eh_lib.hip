@@ -1866,6 +1866,51 @@ static long ensure_desc(eh_beam *b, long n) {
   return EH_OK;
 }
 
+/* a 64-bit hash of bytes, eight at a time in four chains (a byte-wise hash of a
+ * batch's element structs took 6 ms per call, this one 0.5) */
+static uint64_t hash_bytes(const void *p, size_t n, uint64_t seed = 0) {
+  const unsigned char *c = (const unsigned char *)p;
+  uint64_t h[4] = {seed ^ 0x9e3779b97f4a7c15ull, seed ^ 0xbf58476d1ce4e5b9ull, seed ^ 0x94d049bb133111ebull, seed + n};
+  size_t i = 0;
+  for (; i + 32 <= n; i += 32)
+    for (int k = 0; k < 4; k++) {
+      uint64_t w;
+      std::memcpy(&w, c + i + 8 * k, 8);
+      h[k] = (h[k] ^ w) * 0x9fb21c651e98df25ull;
+      h[k] ^= h[k] >> 32;
+    }
+  for (int k = 0; i < n; k = (k + 1) & 3) {
+    uint64_t w = 0;
+    const size_t m = std::min((size_t)8, n - i);
+    std::memcpy(&w, c + i, m);
+    h[k] = (h[k] ^ w) * 0x9fb21c651e98df25ull;
+    h[k] ^= h[k] >> 32;
+    i += m;
+  }
+  uint64_t r = h[0];
+  for (int k = 1; k < 4; k++) {
+    r = (r ^ h[k]) * 0xd6e8feb86659fd93ull;
+    r ^= r >> 29;
+  }
+  return r;
+}
+
+/* the distinct descriptors among those given to add(), in order of appearance */
+struct eh_distinct {
+  std::vector<eh_desc> list;
+  std::unordered_multimap<uint64_t, int32_t> at;
+  int32_t add(const eh_desc &d) {
+    const uint64_t h = hash_bytes(&d, sizeof d);
+    auto r = at.equal_range(h);
+    for (auto it = r.first; it != r.second; ++it)
+      if (!std::memcmp(&list[it->second], &d, sizeof d))
+        return it->second;
+    at.emplace(h, (int32_t)list.size());
+    list.push_back(d);
+    return (int32_t)list.size() - 1;
+  }
+};
+
 /* point a bend at the first of the field-term blocks equal to its own (every bend
  * appends its block to the pool), so that bends that differ only in where their
  * terms lie get equal descriptors */
@@ -1903,9 +1948,8 @@ static void share_terms(eh_desc &d, const std::vector<eh_fterm> &pool, eh_term_b
 static long upload_fused_descs(eh_beam *b, const std::vector<eh_desc> &hd, const std::vector<eh_fterm> &pool) {
   const long ne = (long)hd.size();
   eh_term_blocks blocks;
-  std::vector<eh_desc> uniq;
+  eh_distinct uniq;
   std::vector<eh_pos> pos(ne);
-  std::unordered_map<std::string, int64_t> seen;
   const int64_t base = (int64_t)sizeof(eh_pos) * ne;
   for (long ie = 0; ie < ne; ie++) {
     eh_desc k;
@@ -1915,15 +1959,9 @@ static long upload_fused_descs(eh_beam *b, const std::vector<eh_desc> &hd, const
     pos[ie].pad_ = 0;
     k.zpos[0] = k.zpos[1] = 0;
     share_terms(k, pool, blocks);
-    std::string key(reinterpret_cast<const char *>(&k), sizeof k);
-    auto it = seen.find(key);
-    if (it == seen.end()) {
-      it = seen.emplace(std::move(key), base + (int64_t)sizeof(eh_desc) * (int64_t)uniq.size()).first;
-      uniq.push_back(k);
-    }
-    pos[ie].off = it->second;
+    pos[ie].off = base + (int64_t)sizeof(eh_desc) * uniq.add(k);
   }
-  const long bytes = (long)base + (long)(sizeof(eh_desc) * uniq.size());
+  const long bytes = (long)base + (long)(sizeof(eh_desc) * uniq.list.size());
   if (b->fused_cap < bytes) {
     if (b->noalloc)
       return fail(EH_ERR_ARG, "the line's %ld positions exceed the static scratch", ne);
@@ -1936,7 +1974,8 @@ static long upload_fused_descs(eh_beam *b, const std::vector<eh_desc> &hd, const
   }
   if (ne) {
     HIPCHK(hipMemcpy(b->d_fused, pos.data(), (size_t)base, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(b->d_fused + base, uniq.data(), sizeof(eh_desc) * uniq.size(), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(b->d_fused + base, uniq.list.data(), sizeof(eh_desc) * uniq.list.size(),
+                     hipMemcpyHostToDevice));
   }
   return EH_OK;
 }
@@ -3769,22 +3808,15 @@ static size_t elem_struct_size(int32_t type) {
   }
 }
 
-/* FNV-1a over every element struct of every variant, and P_central */
+/* a hash of every element struct of every variant, and P_central */
 static uint64_t beamlines_hash(EH_ELEMENT_LIST *const *bl, long nvar, long ne, double Pc) {
-  uint64_t h = 1469598103934665603ull;
-  auto mix = [&](const void *p, size_t n) {
-    const unsigned char *c = (const unsigned char *)p;
-    for (size_t i = 0; i < n; i++) {
-      h ^= c[i];
-      h *= 1099511628211ull;
-    }
-  };
-  mix(&Pc, sizeof Pc);
+  uint64_t h = hash_bytes(&Pc, sizeof Pc);
   for (long v = 0; v < nvar; v++)
     for (long e = 0; e < ne; e++) {
-      mix(&bl[v][e].type, sizeof(int32_t));
-      if (bl[v][e].p_elem)
-        mix(bl[v][e].p_elem, elem_struct_size(bl[v][e].type));
+      const EH_ELEMENT_LIST &el = bl[v][e];
+      h = hash_bytes(&el.type, sizeof(int32_t), h);
+      if (el.p_elem)
+        h = hash_bytes(el.p_elem, elem_struct_size(el.type), h);
     }
   return h;
 }
@@ -4115,6 +4147,40 @@ static int32_t pool_push(eh_desc d, const std::vector<eh_fterm> &ft, std::vector
   return (int32_t)pool.size() - 1;
 }
 
+/* whether pool entry q is descriptor d with field terms ft (pool_push's shift
+ * undone) */
+static bool pool_equal(const eh_desc &d, const std::vector<eh_fterm> &ft, const eh_desc &q,
+                       const std::vector<eh_fterm> &terms) {
+  eh_desc k;
+  std::memcpy(&k, &q, sizeof k);
+  if (!ft.empty()) {
+    if (k.type != EH_T_CSBEND)
+      return false;
+    const int32_t shift = k.csb_fx0 - d.csb_fx0;
+    if (shift < 0 || (size_t)shift + ft.size() > terms.size() ||
+        std::memcmp(terms.data() + shift, ft.data(), sizeof(eh_fterm) * ft.size()))
+      return false;
+    k.csb_fx0 -= shift;
+    k.csb_fy0 -= shift;
+    if (k.csb_dense) {
+      k.csb_dx0 -= shift;
+      k.csb_dy0 -= shift;
+    }
+  }
+  return !std::memcmp(&k, &d, sizeof k);
+}
+
+static bool same_amp(const EH_MAXAMP *a, const EH_MAXAMP *b) {
+  return a == b || (a && b && !std::memcmp(a, b, sizeof *a));
+}
+
+/* whether two positions give one element struct the same descriptor */
+static bool same_context(const eh_ctx &a, const eh_ctx &b) {
+  return a.Po == b.Po && a.z_start == b.z_start && a.z_end == b.z_end && same_amp(a.ap[0], b.ap[0]) &&
+         same_amp(a.ap[1], b.ap[1]) && !std::memcmp(a.post_x, b.post_x, sizeof a.post_x) &&
+         !std::memcmp(a.post_y, b.post_y, sizeof a.post_y) && !std::memcmp(a.post_on, b.post_on, sizeof a.post_on);
+}
+
 /* the descriptor pool of all variants, de-duplicated by content (descriptor
  * bytes and field terms), with idx[v*ne + e] the descriptor of element e of
  * variant v.  RF cavities whose fiducial is still pending get a MARK placeholder
@@ -4122,17 +4188,30 @@ static int32_t pool_push(eh_desc d, const std::vector<eh_fterm> &ft, std::vector
  * code only (no HIP calls), so that tests can run it on the CPU. */
 static long batch_tables(EH_ELEMENT_LIST *const *beamlines, long nvar, long ne, double Pc,
                          std::vector<eh_desc> &pool, std::vector<eh_fterm> &terms, std::vector<int32_t> &idx) {
-  std::unordered_map<std::string, int32_t> seen;
+  std::unordered_multimap<uint64_t, int32_t> seen;
   pool.clear();
   terms.clear();
   idx.assign((size_t)nvar * ne, 0);
-  std::vector<eh_ctx> ctx;
+  std::vector<eh_ctx> ctx, ctx0;
+  std::vector<eh_fterm> ft;
   for (long v = 0; v < nvar; v++) {
     const EH_ELEMENT_LIST *bl = beamlines[v];
     line_contexts(bl, ne, Pc, ctx);
+    if (v == 0)
+      ctx0 = ctx;
     for (long e = 0; e < ne; e++) {
+      /* the same struct in the same place and between the same apertures as in
+       * variant 0 gives the same descriptor, without building it */
+      if (v > 0 && bl[e].type == beamlines[0][e].type && bl[e].type != EH_T_RFCA &&
+          same_context(ctx[e], ctx0[e]) &&
+          (bl[e].p_elem == beamlines[0][e].p_elem ||
+           (bl[e].p_elem && beamlines[0][e].p_elem &&
+            !std::memcmp(bl[e].p_elem, beamlines[0][e].p_elem, elem_struct_size(bl[e].type))))) {
+        idx[(size_t)v * ne + e] = idx[e];
+        continue;
+      }
       eh_desc d;
-      std::vector<eh_fterm> ft;
+      ft.clear();
       long r;
       if (rf_pending(bl + e)) {
         std::memset(&d, 0, sizeof d);
@@ -4143,16 +4222,19 @@ static long batch_tables(EH_ELEMENT_LIST *const *beamlines, long nvar, long ne, 
         r = build_desc(&d, bl + e, ctx[e], ft);
       if (r < 0)
         return r;
-      std::string key((const char *)&d, sizeof d);
-      key.append((const char *)ft.data(), sizeof(eh_fterm) * ft.size());
-      auto it = seen.find(key);
-      if (it != seen.end() && bl[e].type != EH_T_RFCA) {
-        idx[(size_t)v * ne + e] = it->second;
-      } else {
-        int32_t id = pool_push(d, ft, pool, terms);
-        seen.emplace(key, id);
-        idx[(size_t)v * ne + e] = id;
+      const uint64_t h = hash_bytes(ft.data(), sizeof(eh_fterm) * ft.size(), hash_bytes(&d, sizeof d));
+      int32_t found = -1;
+      if (bl[e].type != EH_T_RFCA) {
+        auto range = seen.equal_range(h);
+        for (auto it = range.first; it != range.second && found < 0; ++it)
+          if (pool_equal(d, ft, pool[it->second], terms))
+            found = it->second;
       }
+      if (found < 0) {
+        found = pool_push(d, ft, pool, terms);
+        seen.emplace(h, found);
+      }
+      idx[(size_t)v * ne + e] = found;
     }
   }
   return EH_OK;
@@ -4256,6 +4338,13 @@ extern "C" long eh_batch_track(eh_batch *b, EH_ELEMENT_LIST *const *beamlines, l
       b->rad = b->rad || !eh_lean_capable(d);
     b->kmp_idx = any_kick ? std::make_shared<const std::vector<int32_t>>(idx) : nullptr;
   }
+  /* room for the descriptors that replace pending RF cavities, so that those are
+   * appended to the tables on the device */
+  size_t room = pool.size();
+  for (long e : rf_elems)
+    for (long v = 0; v < b->nvar; v++)
+      room += rf_pending(beamlines[v] + e) ? (size_t)ne : 0;
+  room = std::min(room, pool.size() + rf_elems.size() * rf_elems.size() * (size_t)b->nvar);
   auto upload_tables = [&]() -> long {
     b->tables_hash = 0; /* valid again only once this call completes */
     if (b->d_pool)
@@ -4267,7 +4356,7 @@ extern "C" long eh_batch_track(eh_batch *b, EH_ELEMENT_LIST *const *beamlines, l
     b->d_pool = nullptr;
     b->d_terms = nullptr;
     b->d_desc_idx = nullptr;
-    HIPCHK(hipMalloc(&b->d_pool, sizeof(eh_desc) * pool.size()));
+    HIPCHK(hipMalloc(&b->d_pool, sizeof(eh_desc) * room));
     HIPCHK(hipMemcpy(b->d_pool, pool.data(), sizeof(eh_desc) * pool.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMalloc(&b->d_terms, sizeof(eh_fterm) * (terms.size() + 1)));
     if (!terms.empty())
@@ -4335,12 +4424,20 @@ extern "C" long eh_batch_track(eh_batch *b, EH_ELEMENT_LIST *const *beamlines, l
         if (r < 0)
           return r;
       }
+      const size_t had = pool.size();
       r = batch_rf_update(beamlines, b->nvar, ne, er, Pc, pool, terms, idx);
       if (r < 0)
         return r;
-      r = upload_tables();
-      if (r < 0)
-        return r;
+      if (pool.size() > room) { /* more positions share a cavity than there are cavities */
+        room = pool.size();
+        r = upload_tables();
+        if (r < 0)
+          return r;
+      } else {
+        HIPCHK(hipMemcpy(b->d_pool + had, pool.data() + had, sizeof(eh_desc) * (pool.size() - had),
+                         hipMemcpyHostToDevice));
+        HIPCHK(hipMemcpy(b->d_desc_idx, idx.data(), sizeof(int32_t) * idx.size(), hipMemcpyHostToDevice));
+      }
       e = (int)er;
     }
   }
@@ -4444,8 +4541,7 @@ struct eh_apos {
 /* the table of all variants' positions followed by the distinct descriptors */
 static std::vector<char> adj_table(const std::vector<eh_desc> &hd, const std::vector<eh_fterm> &pool) {
   std::vector<eh_apos> pos(hd.size());
-  std::vector<eh_desc> uniq;
-  std::unordered_map<std::string, int64_t> seen;
+  eh_distinct uniq;
   eh_term_blocks blocks;
   const int64_t base = (int64_t)(sizeof(eh_apos) * hd.size());
   for (size_t i = 0; i < hd.size(); i++) {
@@ -4458,17 +4554,11 @@ static std::vector<char> adj_table(const std::vector<eh_desc> &hd, const std::ve
     for (int32_t *s : {&k.adj_pk, &k.adj_pdx, &k.adj_pdy, &k.adj_pfse})
       *s = *s >= 0 ? 0 : -1;
     share_terms(k, pool, blocks);
-    std::string key(reinterpret_cast<const char *>(&k), sizeof k);
-    auto it = seen.find(key);
-    if (it == seen.end()) {
-      it = seen.emplace(std::move(key), base + (int64_t)(sizeof(eh_desc) * uniq.size())).first;
-      uniq.push_back(k);
-    }
-    pos[i].off = it->second;
+    pos[i].off = base + (int64_t)sizeof(eh_desc) * uniq.add(k);
   }
-  std::vector<char> table((size_t)base + sizeof(eh_desc) * uniq.size());
+  std::vector<char> table((size_t)base + sizeof(eh_desc) * uniq.list.size());
   std::memcpy(table.data(), pos.data(), (size_t)base);
-  std::memcpy(table.data() + base, uniq.data(), sizeof(eh_desc) * uniq.size());
+  std::memcpy(table.data() + base, uniq.list.data(), sizeof(eh_desc) * uniq.list.size());
   return table;
 }
 

@@ -109,6 +109,10 @@ class Lattice:
         el = self.elements[i]
         el.params[name] = value
         if self._structs is not None and self._structs[i] is not None:
+            field = S.plain_field(el.type, name, el.params)
+            if field:
+                setattr(self._structs[i], field, value)
+                return
             new = S.make_struct(el.type, el.params)
             if el.type == S.T_CSBEND:
                 new.edgeFlags = self._edge_flags(i)

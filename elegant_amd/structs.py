@@ -195,6 +195,15 @@ ALIASES = {
 }
 
 
+def plain_field(etype, name, params):
+    """the struct field a parameter sets and nothing else does, if it is a double
+    (None otherwise: another spelling of it may be among the params, say)"""
+    key = _PLAIN.get((etype, name))
+    if key is not None and sum(1 for k in params if k.upper() == name) == 1:
+        return key
+    return None
+
+
 def make_struct(etype, params):
     """Build the ctypes struct for an element from elegant-style parameters."""
     cls = STRUCT_OF[etype]
@@ -214,3 +223,9 @@ def make_struct(etype, params):
     for k, v in vals.items():
         setattr(s, k, v)
     return s
+
+
+# strengths and offsets as the gradients name them: one double field each
+_PLAIN = {(t, n): n.lower() for t, names in ((T_KQUAD, ("K1", "DX", "DY")), (T_KSEXT, ("K2", "DX", "DY")),
+                                             (T_KOCT, ("K3", "DX", "DY")), (T_KQUSE, ("K1", "DX", "DY")),
+                                             (T_CSBEND, ("K1", "FSE"))) for n in names}
