@@ -1758,19 +1758,19 @@ EH_HD int eh_sweeps(eh_p6 &p, const eh_desc &d, int pi, const double *__restrict
  * survives, else the loss stage (EH_STAGE_ELEMENT possibly with
  * EH_STAGE_INHERIT). */
 template <bool RAD>
-EH_HD int eh_apply_element_t(eh_p6 &p, const eh_desc &d, int pass, const eh_fterm *__restrict__ terms,
+EH_HD int eh_apply_element_k(eh_p6 &p, int type, const eh_desc &d, int pass, const eh_fterm *__restrict__ terms,
                              const double *__restrict__ zp) {
   const int pi = pass > 0 ? 1 : 0;
   bool lost = false;
   int flag = 0;
-  if constexpr (!RAD) {
-    if (d.full_only)
-      return EH_STAGE_REFUSED;
+  switch (type) {
+  case 1: { /* DRIF; its limits are read along with its length */
+    const double L = d.length, T = d.T11, sx = d.sw_x[pi], sy = d.sw_y[pi];
+    eh_drif(p, L, T);
+    if (eh_fabs(p.x) <= sx && eh_fabs(p.y) <= sy)
+      return -1;
+    return eh_sweeps<RAD>(p, d, pi, zp);
   }
-  switch (d.type) {
-  case 1: /* DRIF */
-    eh_drif(p, d.length, d.T11);
-    break;
   case 2: /* EDRIFT */
     eh_edrift(p, d.length);
     break;
@@ -1824,6 +1824,22 @@ EH_HD int eh_apply_element_t(eh_p6 &p, const eh_desc &d, int pass, const eh_fter
     return -1;
   return eh_sweeps<RAD>(p, d, pi, zp);
 }
+
+/* the same for a descriptor whose line nobody has checked: the lean map refuses
+ * what only the full one carries */
+template <bool RAD>
+EH_HD int eh_apply_element_t(eh_p6 &p, const eh_desc &d, int pass, const eh_fterm *__restrict__ terms,
+                             const double *__restrict__ zp) {
+  if constexpr (!RAD) {
+    if (d.full_only)
+      return EH_STAGE_REFUSED;
+  }
+  return eh_apply_element_k<RAD>(p, d.type, d, pass, terms, zp);
+}
+
+/* whether an element type counts as particle-element units: all but MARK and
+ * MAXAMP (eh_desc.counted) */
+EH_HD int eh_counted(int type) { return type != 0 && type != 8; }
 
 /* where and how a particle was lost inside a fused span, in one word: element
  * ee of pass p0 + dpass (nelem elements per pass) at stage st (EH_STAGE_*; the

@@ -60,3 +60,27 @@ def test_rows_by_pointer(ehlib, oracle_mod, n):
     assert_rows_identical(store[place, :S.NPROP], ref, na, nref, "by pointer")
     assert (store[:, S.NPROP:] == -7.0).all()
     beam.free()
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 128, 129, 200])
+def test_line_lengths(ehlib, oracle_mod, n):
+    """positions are read 64 at a time: lines of about that many elements and of
+    multiples, spans that begin inside a line (after a cavity), losses all along"""
+    rng = np.random.default_rng(n)
+    kinds = [("DRIF", dict(L=0.3)), ("KQUAD", dict(L=0.2, K1=0.6, N_KICKS=2)), ("EDRIFT", dict(L=0.2)), ("MARK", {}),
+             ("KSEXT", dict(L=0.1, K2=4.0, N_KICKS=2)), ("MAXAMP", dict(X_MAX=4e-3, Y_MAX=3e-3)),
+             ("RFCA", dict(L=0.1, VOLT=1e5, FREQ=5e8, PHASE=90.0))]
+    els = [Element("%s%d" % (kinds[k][0], k), kinds[k][0], **kinds[k][1])
+           for k in np.append(rng.integers(0, 6, n - 1), 0 if n < 63 else 6)]
+    rng.shuffle(els)
+    rows = rows_of(400, 1e-3)
+    ref, nref, _, _ = oracle_mod.do_tracking(rows, Lattice(els), 3, Po)
+    for turns in (16, 1):
+        beam = tracking.Beam(rows)
+        na, _, st = tracking.track(beam, Lattice(els), 3, Po, mode="fused", turns_per_launch=turns)
+        assert_rows_identical(beam.download(), ref, na, nref, "fused n=%d" % n)
+        beam.free()
+    batch = tracking.Batch([rows, rows[:65]])
+    batch.track([Lattice(els), Lattice(els)], 3, Po, span_elements=70)
+    assert_rows_identical(batch.download(0), ref, batch.n_alive(0), nref, "batch n=%d" % n)
+    batch.free()
