@@ -84,3 +84,18 @@ def test_line_lengths(ehlib, oracle_mod, n):
     batch.track([Lattice(els), Lattice(els)], 3, Po, span_elements=70)
     assert_rows_identical(batch.download(0), ref, batch.n_alive(0), nref, "batch n=%d" % n)
     batch.free()
+
+
+@pytest.mark.parametrize("counts", [[1], [0, 1, 64, 65], [300000, 5, 0, 129]])
+def test_batch_rows(ehlib, oracle_mod, counts):
+    """a variant's rows go up and down through memory that all variants share: chunks,
+    empty variants, losses in some of them, a cavity's fiducial in each"""
+    lat = [Lattice(line().elements + [Element("RF", "RFCA", L=0.1, VOLT=1e5, FREQ=5e8, PHASE=90.0)]) for _ in counts]
+    ref_lat = [Lattice(line().elements + [Element("RF", "RFCA", L=0.1, VOLT=1e5, FREQ=5e8, PHASE=90.0)]) for _ in counts]
+    rows = [rows_of(n, (6e-3, 1e-4)[v % 2]) if n else np.zeros((0, S.NPROP)) for v, n in enumerate(counts)]
+    batch = tracking.Batch(rows)
+    batch.track(lat, 2, Po)
+    for v in reversed(range(len(counts))):
+        ref, nref, _, _ = oracle_mod.do_tracking(rows[v], ref_lat[v], 2, Po)
+        assert_rows_identical(batch.download(v), ref, batch.n_alive(v), nref, "variant %d" % v)
+    batch.free()
