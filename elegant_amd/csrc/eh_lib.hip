@@ -1425,10 +1425,10 @@ extern "C" long eh_beam_upload(eh_beam *b, double **coord, long n_part) {
 /* Occupancy target for the tracking kernels: five wavefronts per SIMD, 96 VGPRs.
  * The regular integrators are bound by instruction issue, which four or five
  * wavefronts fill; a sixth only costs spills around them.  Kernel time in ms at 3,
- * 4, 5, 6 and 8 wavefronts: MBA ring, 2 turns, 1e6 particles 149.6, 148.7, 147.4,
- * 147.6, 160.5; 30401 particles (one wavefront per SIMD or none) 17.7, 17.1, 17.4,
- * 17.5, 23.0; with radiation, 5e4 particles, 1 turn 11.7, 11.9, 11.7, 13.2, 17.4;
- * FODO ring, 1e4 particles, 40 turns 11.2, 11.2, 11.2, 12.3, 14.6. */
+ * 4, 5 and 6 wavefronts: MBA ring, 2 turns, 1e6 particles 143.7, 139.4, 137.3, 139.5;
+ * 30401 particles (one wavefront per SIMD or none) 15.6, 16.0, 15.7, 17.2; with
+ * radiation, 5e4 particles, 1 turn 11.0, 11.1, 11.2, 11.7; FODO ring, 1e4 particles,
+ * 40 turns 10.1, 10.0, 10.0, 11.9. */
 #define EH_TRACK_WAVES __attribute__((amdgpu_waves_per_eu(5)))
 
 __device__ __forceinline__ eh_p6 load_p(const eh_soa a, long i) {
@@ -2369,7 +2369,7 @@ static long check_missing(const eh_rows &w, const char *what);
 
 /* the TMEAN fiducial: the arrival times in the reference's row order from the
  * device; their Kahan sum is a serial chain, which the host runs.  A batch of 12
- * variants of about 16000 particles spent 18.5 ms outside its kernels when the host
+ * variants, 3.2e5 particles, spent 18.5 ms outside its kernels when the host
  * gathered and divided, 12.1 now. */
 static long tmean_fiducial(const eh_rows &w, double sOffset, double p0, double *tFid) {
   const long n = w.na;
@@ -3965,8 +3965,8 @@ extern "C" long eh_batch_upload(eh_batch *b, long v, const double *flat, long n)
     return fail(EH_ERR_ARG, "eh_batch_upload: bad arguments");
   if (b->cur != 0 || b->n_lost)
     return fail(EH_ERR_STATE, "eh_batch_upload: upload every variant before tracking");
-  /* as upload_rows, through the other buffer.  12 variants of about 16000
-   * particles up: 5.7 ms when the host took the rows apart, 1.7 now; down 3.2 and
+  /* as upload_rows, through the other buffer.  12 variants, 3.2e5
+   * particles, up: 5.7 ms when the host took the rows apart, 1.7 now; down 3.2 and
    * 2.2. */
   std::lock_guard<std::mutex> one(b->rows_mx);
   char *buf = (char *)b->mem + b->region;
