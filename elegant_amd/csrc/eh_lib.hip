@@ -848,14 +848,17 @@ static long build_element(eh_desc *d, const EH_ELEMENT_LIST *e, const eh_ctx &c,
 
 /* the head's limits: what the sweeps after the element clear without a look at
  * their kind (a plain MAXAMP's limits, or every finite coordinate where there is
- * none; nothing for elliptical ones), and the in-element limits */
+ * none; nothing for elliptical ones), and the in-element limits.  A limit may be
+ * infinite, which an infinite coordinate would pass: none is above the largest
+ * double, and the regular path's none above what its quotients take. */
 static void head_limits(eh_desc *d) {
+  auto up_to = [](double limit, double most) { return limit > 0 ? std::min(limit, most) : most; };
   for (int pi = 0; pi < 2; pi++) {
     const bool on = d->post_ap[pi] != 0;
-    d->sw_x[pi] = d->post_ell[pi] ? -1.0 : on && d->post_xmax[pi] > 0 ? d->post_xmax[pi] : EH_DBL_MAX;
-    d->sw_y[pi] = d->post_ell[pi] ? -1.0 : on && d->post_ymax[pi] > 0 ? d->post_ymax[pi] : EH_DBL_MAX;
-    d->reg_apx[pi] = d->ap_xmax[pi] > 0 ? d->ap_xmax[pi] : 0x1p60;
-    d->reg_apy[pi] = d->ap_ymax[pi] > 0 ? d->ap_ymax[pi] : 0x1p60;
+    d->sw_x[pi] = d->post_ell[pi] ? -1.0 : up_to(on ? d->post_xmax[pi] : 0, EH_DBL_MAX);
+    d->sw_y[pi] = d->post_ell[pi] ? -1.0 : up_to(on ? d->post_ymax[pi] : 0, EH_DBL_MAX);
+    d->reg_apx[pi] = up_to(d->ap_xmax[pi], 0x1p60);
+    d->reg_apy[pi] = up_to(d->ap_ymax[pi], 0x1p60);
   }
 }
 

@@ -144,6 +144,43 @@ def test_who_is_regular(name):
     assert out.sum() > 20 and not taken[out].any()
 
 
+UNBOUNDED = [(np.inf, 0.02), (0.02, np.inf), (np.inf, np.inf), (np.nan, 0.02), (np.finfo(float).max, 0.02)]
+
+
+def overflowing():
+    """an aperture's limit may be infinite, a coordinate that overflows is lost all
+    the same: (line, rows) per limits, drifts and a bend whose entry is at 1e308"""
+    rows = np.zeros((4, S.NPROP))
+    rows[1, 1] = rows[2, 3] = 1e307
+    rows[3, 0] = rows[3, 2] = 1e308
+    rows[:, 6] = np.arange(1, 5)
+    for x, y in UNBOUNDED:
+        for els in ([Element("D", "EDRIFT", L=1000.0)], [Element("D", "DRIF", L=1000.0), ELEMENTS["bend"][0]]):
+            yield Lattice([Element("AP", "MAXAMP", X_MAX=x, Y_MAX=y)] + els), rows, "%g %g" % (x, y)
+
+
+def test_infinite_limits_keep_no_infinite_coordinate():
+    for lat, rows, what in overflowing():
+        r, out6, lpass, _ = _host_track([rows], [lat], 1, Po, None, 1)
+        ref, n, _, _ = oracle.do_tracking(rows, lat, 1, Po)
+        alive = set(np.flatnonzero(lpass == -1) + 1)
+        assert r == n and alive == set(ref[:n, 6].astype(int)), what
+        check(out6[ref[:n, 6].astype(int) - 1], ref[:n, :6], what)
+
+
+@pytest.mark.gpu
+def test_infinite_limits_on_the_gpu(ehlib):
+    for lat, rows, what in overflowing():
+        ref, nref, _, _ = oracle.do_tracking(rows, lat, 1, Po)
+        for mode in ("fused", "plain"):
+            beam = tracking.Beam(rows)
+            n, _, _ = tracking.track(beam, lat, 1, Po, mode=mode)
+            got = beam.download()
+            beam.free()
+            assert n == nref, what
+            check(got, ref, what + " " + mode)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", sorted(ELEMENTS))
 def test_gpu_matches_oracle(ehlib, name):
