@@ -3834,6 +3834,17 @@ extern "C" long eh_diag_copy(long n, int reps) {
 #include <string>
 #include <unordered_map>
 
+/* The beamlines a batch's tables on the device were made from: P_central and every
+ * element's type and struct, kept as bytes and compared as bytes (a hash alone took
+ * edited beamlines for the kept ones: the sign of both limits of a MAXAMP changed).
+ * A struct of a later variant that equals variant 0's is a mark of one byte; error
+ * seeds differ in some of their magnets only. */
+struct eh_kept_lines {
+  double Pc = 0;
+  long nvar = 0, ne = 0;
+  std::vector<char> bytes;
+};
+
 struct eh_batch {
   long nvar = 0;
   std::vector<long> n_v, id_off, region_off;
@@ -3858,8 +3869,7 @@ struct eh_batch {
   long launches = 0;
   int n_cu = 256;
   /* descriptor tables of the last call, reused while the beamlines are unchanged */
-  uint64_t tables_hash = 0;
-  long tables_ne = 0;
+  eh_kept_lines tables_of; /* ne is 0 while the tables serve no later call */
   bool rad = false;    /* some descriptor of the pool radiates */
   eh_kmp_tab kmp_pool; /* kick-multipole records of the descriptor pool */
   eh_kmp_idx kmp_idx;  /* variant * ne + element -> pool entry */
@@ -3899,17 +3909,50 @@ static size_t elem_struct_size(int32_t type) {
   }
 }
 
-/* a hash of every element struct of every variant, and P_central */
-static uint64_t beamlines_hash(EH_ELEMENT_LIST *const *bl, long nvar, long ne, double Pc) {
-  uint64_t h = hash_bytes(&Pc, sizeof Pc);
+enum { EH_KEPT_NULL = 0, EH_KEPT_FIRST = 1, EH_KEPT_OWN = 2 };
+
+/* how element e of variant v is kept */
+static char kept_as(EH_ELEMENT_LIST *const *bl, long v, long e) {
+  const EH_ELEMENT_LIST &a = bl[v][e], &f = bl[0][e];
+  if (!a.p_elem)
+    return EH_KEPT_NULL;
+  const bool first = v > 0 && a.type == f.type && f.p_elem &&
+                     (a.p_elem == f.p_elem || !std::memcmp(a.p_elem, f.p_elem, elem_struct_size(a.type)));
+  return first ? EH_KEPT_FIRST : EH_KEPT_OWN;
+}
+
+static void keep_lines(eh_kept_lines &k, EH_ELEMENT_LIST *const *bl, long nvar, long ne, double Pc) {
+  k.Pc = Pc;
+  k.nvar = nvar;
+  k.ne = ne;
+  k.bytes.clear();
+  auto put = [&](const void *p, size_t n) { k.bytes.insert(k.bytes.end(), (const char *)p, (const char *)p + n); };
   for (long v = 0; v < nvar; v++)
     for (long e = 0; e < ne; e++) {
-      const EH_ELEMENT_LIST &el = bl[v][e];
-      h = hash_bytes(&el.type, sizeof(int32_t), h);
-      if (el.p_elem)
-        h = hash_bytes(el.p_elem, elem_struct_size(el.type), h);
+      const char how = kept_as(bl, v, e);
+      put(&how, 1);
+      put(&bl[v][e].type, sizeof(int32_t));
+      if (how == EH_KEPT_OWN)
+        put(bl[v][e].p_elem, elem_struct_size(bl[v][e].type));
     }
-  return h;
+}
+
+/* whether the beamlines are those kept; variant 0's structs come first, so that a
+ * mark stands for bytes already found equal */
+static bool lines_kept(const eh_kept_lines &k, EH_ELEMENT_LIST *const *bl, long nvar, long ne, double Pc) {
+  if (std::memcmp(&k.Pc, &Pc, sizeof Pc) || k.nvar != nvar || k.ne != ne)
+    return false;
+  const char *p = k.bytes.data();
+  for (long v = 0; v < nvar; v++)
+    for (long e = 0; e < ne; e++) {
+      const char how = kept_as(bl, v, e);
+      const size_t own = how == EH_KEPT_OWN ? elem_struct_size(bl[v][e].type) : 0;
+      if (*p != how || std::memcmp(p + 1, &bl[v][e].type, sizeof(int32_t)) ||
+          (own && std::memcmp(p + 1 + sizeof(int32_t), bl[v][e].p_elem, own)))
+        return false;
+      p += 1 + sizeof(int32_t) + own;
+    }
+  return true;
 }
 
 extern "C" eh_batch *eh_batch_create(long nvar, const long *n_particles) {
@@ -4272,9 +4315,9 @@ static long batch_rf_update(EH_ELEMENT_LIST *const *beamlines, long nvar, long n
 /* the device tables of the last call can serve this one only if the beamlines
  * are byte-for-byte unchanged and no RF cavity still waits for its fiducial
  * (whose placeholder the pass-0 stop has to replace in the host copy) */
-static bool batch_tables_reusable(bool have_tables, long tables_ne, uint64_t tables_hash,
-                                  EH_ELEMENT_LIST *const *beamlines, long nvar, long ne, uint64_t hash) {
-  if (!have_tables || tables_ne != ne || tables_hash != hash)
+static bool batch_tables_reusable(const eh_kept_lines &kept, EH_ELEMENT_LIST *const *beamlines, long nvar, long ne,
+                                  double Pc) {
+  if (!lines_kept(kept, beamlines, nvar, ne, Pc))
     return false;
   for (long v = 0; v < nvar; v++)
     for (long e = 0; e < ne; e++)
@@ -4327,9 +4370,7 @@ extern "C" long eh_batch_track(eh_batch *b, EH_ELEMENT_LIST *const *beamlines, l
   for (long e = 0; e < ne; e++)
     if (beamlines[0][e].type == EH_T_RFCA)
       rf_elems.push_back(e);
-  const uint64_t hash = beamlines_hash(beamlines, b->nvar, ne, Pc);
-  const bool reuse =
-      batch_tables_reusable(b->d_pool != nullptr, b->tables_ne, b->tables_hash, beamlines, b->nvar, ne, hash);
+  const bool reuse = b->d_pool && batch_tables_reusable(b->tables_of, beamlines, b->nvar, ne, Pc);
   if (!reuse) {
     long r = batch_tables(beamlines, b->nvar, ne, Pc, pool, terms, idx);
     if (r < 0)
@@ -4352,7 +4393,7 @@ extern "C" long eh_batch_track(eh_batch *b, EH_ELEMENT_LIST *const *beamlines, l
       room += rf_pending(beamlines[v] + e) ? (size_t)ne : 0;
   room = std::min(room, pool.size() + rf_elems.size() * rf_elems.size() * (size_t)b->nvar);
   auto upload_tables = [&]() -> long {
-    b->tables_hash = 0; /* valid again only once this call completes */
+    b->tables_of.ne = 0; /* valid again only once this call completes */
     if (b->d_pool)
       HIPCHK(hipFree(b->d_pool));
     if (b->d_terms)
@@ -4501,8 +4542,8 @@ extern "C" long eh_batch_track(eh_batch *b, EH_ELEMENT_LIST *const *beamlines, l
   for (long v = 0; v < b->nvar; v++)
     alive += b->alive_v[v];
   /* the tables now on the device describe the beamlines as they stand (RF fiducials set) */
-  b->tables_hash = beamlines_hash(beamlines, b->nvar, ne, Pc);
-  b->tables_ne = ne;
+  if (!reuse)
+    keep_lines(b->tables_of, beamlines, b->nvar, ne, Pc);
   if (stats) {
     stats->particle_element_turns = (double)cnt[3];
     stats->kernel_ms = b->kernel_ms - ms0;

@@ -84,13 +84,22 @@ static bool same_desc(const eh_desc &got, const std::vector<eh_fterm> &terms, co
   return std::memcmp(terms.data() + shift, ref_terms.data(), sizeof(eh_fterm) * ref_terms.size()) == 0;
 }
 
+/* whether tables made from the first beamlines would serve a call with the
+ * second */
+extern "C" int bh_tables_serve(EH_ELEMENT_LIST *const *made_from, EH_ELEMENT_LIST *const *call, long nvar, long ne,
+                               double Pc_made, double Pc_call) {
+  eh_kept_lines kept;
+  keep_lines(kept, made_from, nvar, ne, Pc_made);
+  return batch_tables_reusable(kept, call, nvar, ne, Pc_call);
+}
+
 /* Runs the table sequence of eh_batch_track on the host: batch_tables, then for
  * each RF cavity position with a pending fiducial in some variant, a fiducial
  * set from T_REFERENCE-like data (phase_fiducial = -2 pi f * t_set[v]) and
  * batch_rf_update.  Then every (variant, position) of the result is compared
  * with a descriptor built afresh for that position.  Returns the number of
  * mismatching entries, or a negative code.  reusable_before/after report
- * batch_tables_reusable with the tables' own hash before and after the fiducials
+ * batch_tables_reusable for the beamlines as they are before and after the fiducials
  * were set. */
 extern "C" long bh_tables(EH_ELEMENT_LIST *const *beamlines, long nvar, long ne, double Pc, const double *t_set,
                           int32_t *reusable_before, int32_t *reusable_after, int32_t *n_pool) {
@@ -100,8 +109,9 @@ extern "C" long bh_tables(EH_ELEMENT_LIST *const *beamlines, long nvar, long ne,
   long r = batch_tables(beamlines, nvar, ne, Pc, pool, terms, idx);
   if (r < 0)
     return r;
-  uint64_t h0 = beamlines_hash(beamlines, nvar, ne, Pc);
-  *reusable_before = batch_tables_reusable(true, ne, h0, beamlines, nvar, ne, h0);
+  eh_kept_lines kept;
+  keep_lines(kept, beamlines, nvar, ne, Pc);
+  *reusable_before = batch_tables_reusable(kept, beamlines, nvar, ne, Pc);
   for (long er = 0; er < ne; er++) {
     bool pending = false;
     for (long v = 0; v < nvar; v++)
@@ -123,8 +133,8 @@ extern "C" long bh_tables(EH_ELEMENT_LIST *const *beamlines, long nvar, long ne,
     if (r < 0)
       return r;
   }
-  uint64_t h1 = beamlines_hash(beamlines, nvar, ne, Pc);
-  *reusable_after = batch_tables_reusable(true, ne, h1, beamlines, nvar, ne, h1);
+  keep_lines(kept, beamlines, nvar, ne, Pc);
+  *reusable_after = batch_tables_reusable(kept, beamlines, nvar, ne, Pc);
   *n_pool = (int32_t)pool.size();
   long bad = 0;
   std::vector<eh_ctx> ctx;

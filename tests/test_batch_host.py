@@ -174,6 +174,46 @@ def test_tables_after_rf_stop_match_fresh_descriptors(case):
                 assert s.fiducial_seen == 1
 
 
+EDITS = [(-1.0, -1.0), (-1.0, 1.0), (2.0, 2.0), (1.5, 1.5), (0.5, 2.0), (1.0, 1.0 + 2.0 ** -52)]
+
+
+@pytest.mark.parametrize("variant", [0, 1])
+def test_edited_beamlines_get_new_tables(variant):
+    """every pair of neighbouring doubles of every struct edited by a sign or a power of
+    two (edits that some hashes of the bytes do not see); the reference momentum; and
+    the beamlines put back"""
+    def mk():
+        els = [Element("AP", "MAXAMP", X_MAX=0.01, Y_MAX=0.008), Element("D", "DRIF", L=0.5), Element("M", "MARK"),
+               Element("Q", "KQUAD", L=0.25, K1=0.8, N_KICKS=8, DX=1e-5, DY=2e-5, FSE=1e-3),
+               Element("B", "CSBEND", L=0.8, ANGLE=0.03, K1=-0.3, N_KICKS=16, E1=0.01, E2=0.02, HGAP=0.01),
+               Element("AQ", "MAXAMP", X_MAX=0.01, Y_MAX=0.01)]
+        return [Lattice([*els]), Lattice([*els])]
+
+    h = harness()
+    h.bh_tables_serve.argtypes = [C.c_void_p, C.c_void_p, C.c_long, C.c_long, C.c_double, C.c_double]
+    made, call = mk(), mk()
+    pm, km = _lines(made)
+    pc, kc = _lines(call)
+    ne = len(made[0])
+    serve = lambda P=1000.0: h.bh_tables_serve(pm, pc, 2, ne, 1000.0, P)  # noqa: E731
+    assert serve() and not serve(np.nextafter(1000.0, 0))
+    edits = 0
+    for s in call[variant].structs():
+        if s is None:
+            continue
+        d = np.frombuffer(s, dtype=np.float64)
+        for k in range(len(d) - 1):
+            for edit in EDITS:
+                before = d[k:k + 2].copy()
+                if not (np.isfinite(before).all() and (np.abs(before) > 1e-100).all()):
+                    continue  # integers and unset fields among the doubles
+                d[k:k + 2] *= edit
+                assert not serve(), (type(s).__name__, k, edit)
+                d[k:k + 2] = before
+                edits += 1
+    assert edits >= 6 * len(EDITS) and serve()
+
+
 def _beams(counts, seed0=0, scale=400.0):
     return [configs.mba_beam(c, seed=seed0 + v, scale=scale) if c else np.zeros((0, S.NPROP))
             for v, c in enumerate(counts)]

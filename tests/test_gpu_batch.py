@@ -63,6 +63,38 @@ def test_batch_repeated_calls_reuse_tables():
     assert n == total
 
 
+def test_batch_tables_follow_edited_apertures():
+    """a resident batch tracked again after its apertures were edited, by sign and
+    by scale, sees the new ones"""
+    from elegant_amd.lattice import Element, Lattice
+    print("batch edited apertures", flush=True)
+    Po = configs.p_central_from_mev(3000.0)
+
+    def ring(x, y):
+        return Lattice([Element("AP", "MAXAMP", X_MAX=x, Y_MAX=y), Element("D", "DRIF", L=0.5),
+                        Element("Q", "KQUAD", L=0.2, K1=0.5, N_KICKS=4)])
+
+    rng = np.random.default_rng(5)
+    rows = np.zeros((500, 10))
+    rows[:, :4] = rng.normal(0, [8e-3, 1e-4, 8e-3, 1e-4], (500, 4))
+    rows[:, 6] = np.arange(1, 501)
+    steps = [(-0.01, -0.01), (0.03, 0.03), (0.015, 0.015), (0.01, 0.01), (0.005, 0.005)]
+    lats = [ring(*steps[0]), ring(*steps[0])]
+    batch = tracking.Batch([rows, rows[:100]])
+    expect = [rows, rows[:100]]
+    n = [500, 100]
+    for x, y in steps:
+        for v, lat in enumerate(lats):
+            lat.set_param(0, "X_MAX", x)
+            lat.set_param(0, "Y_MAX", y)
+            r, nv, _, _ = oracle.do_tracking(expect[v][:n[v]], ring(x, y), 1, Po)
+            expect[v], n[v] = np.concatenate([r, expect[v][n[v]:]]), nv
+        batch.track(lats, 1, Po)
+        for v in range(2):
+            assert_rows_identical(batch.download(v), expect[v], batch.n_alive(v), n[v], "limits %g %g" % (x, y))
+    assert n[0] < 400
+
+
 def test_batch_more_elements_on_pass():
     """variants of a ring with MULT, ROTATE and MALIGN: the batched kernel applies
     ON_PASS elements on the absolute pass, as each variant tracked alone does"""
