@@ -68,6 +68,13 @@
 #define EH_REG_QMAX 0.0117
 #define EH_REG_QXMAX 0.05
 #define EH_REG_QMIN 0x1p-340
+/* a bend's angles, where eh_sincos is its short series, and the relative change of
+ * 1 + delta at a radiation kick */
+#define EH_REG_ANGLE 0x1p-4
+#define EH_REG_DLOSS 0x1p-18
+/* what the host leaves for the slopes of a small beam where the design orbit itself
+ * comes near a limit */
+#define EH_REG_OWN 1e-3
 /* dense 5 x 5 field block: the terms a gradient alone leaves, (i, j) = (0, 0..4),
  * (1, 0), (1, 2), (1, 3), (2, 2) */
 #define EH_LIVE_GRADIENT 0x9bfu
@@ -117,7 +124,7 @@ EH_HD bool eh_reg_next_recip(double b, double &rh) {
   const double e = eh_fma(-b, rh, 1.0);
   const double y1 = eh_fma(rh, eh_fma(e, e, e), rh);
   rh = eh_fma(eh_fma(-b, y1, 1.0) + 0x1p-80, y1, y1);
-  return eh_fabs(e) < 0x1p-18;
+  return eh_fabs(e) < EH_REG_DLOSS;
 }
 
 /* The coefficients of the short series, opaque to the compiler on the GPU so that
@@ -427,7 +434,7 @@ EH_HD bool eh_csb_regular(const eh_desc &d, int pi, const eh_fterm *__restrict__
       if (nsub == 8)
         th = d.csb_dshr[j];
       const double ang = th + phi;
-      bad |= !(eh_fabs(ang) < 0x1p-4); /* the short series of eh_sincos */
+      bad |= !(eh_fabs(ang) < EH_REG_ANGLE);
       const double sine = eh_reg_sin(ang, ks), cosi = eh_reg_cos(ang, ks);
       const double yc = eh_reg_recip1(cosi);
       const double tang = eh_reg_div(sine, cosi, yc);

@@ -410,3 +410,14 @@ extern "C" long bh_regular_taken(const double *z, long n, const EH_ELEMENT_LIST 
   }
   return count;
 }
+
+/* which regular path the descriptor of an element asks for (eh_desc.regular), or a
+ * negative code */
+extern "C" long bh_regular_asked(const EH_ELEMENT_LIST *e, double Po) {
+  eh_ctx c = {};
+  c.Po = Po;
+  eh_desc d;
+  std::vector<eh_fterm> terms;
+  const long r = build_desc(&d, e, c, terms);
+  return r < 0 ? r : d.regular;
+}

@@ -144,6 +144,52 @@ def test_who_is_regular(name):
     assert out.sum() > 20 and not taken[out].any()
 
 
+def regular_path(el, P, z):
+    """(whether the element asks for the regular path, how many particles it takes)"""
+    arr, keep = Lattice([el]).c_beamline()
+    z = np.ascontiguousarray(z)
+    taken = np.zeros(len(z), dtype=np.int32)
+    h = harness()
+    h.bh_regular_taken.argtypes = [C.c_void_p, C.c_long, C.c_void_p, C.c_double, C.c_double, C.c_double, C.c_void_p]
+    h.bh_regular_taken.restype = C.c_long
+    h.bh_regular_asked.argtypes = [C.c_void_p, C.c_double]
+    h.bh_regular_asked.restype = C.c_long
+    asked = h.bh_regular_asked(C.cast(arr, C.c_void_p), P)
+    assert asked >= 0
+    return asked > 0, h.bh_regular_taken(z.ctypes.data, len(z), C.cast(arr, C.c_void_p), 0.0, 0.0, P,
+                                         taken.ctypes.data)
+
+
+@pytest.mark.parametrize("rad", [0, 1])
+@pytest.mark.parametrize("order", [2, 4, 6])
+def test_no_bend_asks_for_what_it_cannot_pass(order, rad):
+    """the design orbit swings by the sub-step angles and radiates at every kick: a bend
+    whose swing or energy loss no particle can follow does not ask for the regular path,
+    and one that asks passes a small beam whole"""
+    rng = np.random.default_rng(6)
+    z = rng.standard_normal((64, 6)) * [5e-5, 5e-5, 5e-5, 5e-5, 1e-4, 2e-4]
+    seen = set()
+    for mev in (300.0, 3000.0, 7000.0):
+        for rho in (2.0, 6.4, 25.0, 39.0):
+            for degrees in (0.5, 4.5, 18.0, 40.0):
+                for kicks in (4, 5, 6, 8, 12, 30):
+                    angle = np.radians(degrees)
+                    el = Element("B", "CSBEND", L=rho * angle, ANGLE=angle, N_KICKS=kicks, INTEGRATION_ORDER=order,
+                                 SYNCH_RAD=rad, EDGE1_EFFECTS=0, EDGE2_EFFECTS=0)
+                    asked, n = regular_path(el, configs.p_central_from_mev(mev), z)
+                    assert n == (len(z) if asked else 0), (mev, rho, degrees, kicks, n)
+                    seen.add(asked)
+    assert seen == {False, True}
+
+
+@pytest.mark.parametrize("kick", [0.0, 1e-3, 0.02])
+def test_no_corrector_asks_for_what_it_cannot_pass(kick):
+    z = np.random.default_rng(6).standard_normal((64, 6)) * 5e-5
+    for plane in ("HKICK", "VKICK"):
+        el = Element("Q", "KQUAD", L=0.25, K1=1.0, N_KICKS=8, **{plane: kick})
+        assert regular_path(el, Po, z) == ((True, len(z)) if kick < 0.01 else (False, 0))
+
+
 UNBOUNDED = [(np.inf, 0.02), (0.02, np.inf), (np.inf, np.inf), (np.nan, 0.02), (np.finfo(float).max, 0.02)]
 
 
