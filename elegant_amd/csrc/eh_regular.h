@@ -37,10 +37,18 @@
  * integrator, whose branches also keep the compiler from holding the polynomial
  * constants in scalar registers.  Measured (MI355X, MBA ring, fused, 2 turns): 1e6
  * particles 283 -> 166 ms, 30 401 particles (one wavefront on half of the SIMDs)
- * 48.4 -> 21.4 ms; FODO ring, 1e4 particles, 40 turns 27.2 -> 13.4 ms.  A
- * wavefront with one irregular particle pays for both integrators of that
- * element; on a grid filling the aperture of the MBA ring no particle that is not
- * lost ever leaves the limits below.
+ * 48.4 -> 21.4 ms; FODO ring, 1e4 particles, 40 turns 27.2 -> 13.4 ms.
+ *
+ * A wavefront runs the general integrator as soon as one of its particles is beyond
+ * the limits at an element's entry, and both integrators where one leaves them
+ * inside.  On a grid filling the aperture of the MBA ring no particle that is not
+ * lost ever does; of slopes of 5 mrad rms nearly every wavefront has one.  Kernel
+ * times of short lines of such beams, 2 turns, 4e5 particles: quadrupoles and
+ * sextupoles, 5 mrad, 0.58 ms (0.60 with the general integrators alone, 0.70 when
+ * the other particles of the wavefront went on here); with bends, 3 mrad, 1.51 (1.51,
+ * 1.78); 20 mrad, 1.84 (1.85, 2.45).  1e4 particles, one wavefront alone on its SIMD:
+ * 0.19 (0.20, 0.24), 0.52 (0.48, 0.65) and 0.63 (0.61, 0.77).  Looking again at every
+ * slice would win back 0.03 of the 0.52 and cost regular beams 1 to 3 %.
  *
  * With SYNCH_RAD the momentum changes at every kick; its reciprocal follows by a
  * Newton step from the last one.  MBA ring with radiation and edges, 5e4
@@ -230,6 +238,16 @@ EH_HD eh_reg_slopes eh_reg_m2s(double qx, double qy, double b1s, double rh, doub
   return s;
 }
 
+/* Whether any of the wavefront's particles is beyond the limits at entry.  It needs
+ * the general integrator, which costs the same for all of them: nobody goes on here. */
+EH_HD bool eh_reg_any(bool bad) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __ballot(bad) != 0;
+#else
+  return bad;
+#endif
+}
+
 /* zero, or far above underflow */
 EH_HD bool eh_reg_sized(double ax) { return (ax >= EH_REG_QMIN) | (ax == 0); }
 
@@ -271,13 +289,8 @@ EH_HD bool eh_mult_regular(const eh_desc &d, int pi, double &x_, double &xp_, do
   bool bad = !(b1 >= EH_REG_B1_MIN && b1 <= EH_REG_B1_MAX && eh_fabs(x) <= 10.0 && eh_fabs(y) <= 10.0 &&
                eh_fabs(xp_) <= EH_REG_QMAX && eh_fabs(yp_) <= EH_REG_QMAX && eh_reg_sized(eh_fabs(xp_)) &&
                eh_reg_sized(eh_fabs(yp_)));
-#if defined(__HIP_DEVICE_COMPILE__)
-  if (__ballot(!bad) == 0)
+  if (eh_reg_any(bad))
     return false;
-#else
-  if (bad)
-    return false;
-#endif
   double b1s = b1 * b1, rh = 1.0 / b1, rh2 = rh * rh, hrh = 0.5 * rh;
   double qx, qy;
   {
@@ -389,13 +402,8 @@ EH_HD bool eh_csb_regular(const eh_desc &d, int pi, const eh_fterm *__restrict__
   double b1 = 1 + DP;
   bool bad = !(b1 >= EH_REG_B1_MIN && b1 <= EH_REG_B1_MAX && eh_fabs(xp_) <= EH_REG_QMAX &&
                eh_fabs(yp_) <= EH_REG_QMAX && eh_reg_sized(eh_fabs(yp_)));
-#if defined(__HIP_DEVICE_COMPILE__)
-  if (__ballot(!bad) == 0)
+  if (eh_reg_any(bad))
     return false;
-#else
-  if (bad)
-    return false;
-#endif
   const double rho0 = d.rho0, rho_a = d.rho_actual, r0h = d.rho0_rh, rah = d.rhoa_rh;
   const double apx = d.reg_apx[pi], apy = d.reg_apy[pi];
   const double h0 = d.reg_h[0], h1 = d.reg_h[1], k0 = d.reg_k[0], k1 = d.reg_k[1];

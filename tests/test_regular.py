@@ -190,6 +190,25 @@ def test_no_corrector_asks_for_what_it_cannot_pass(kick):
         assert regular_path(el, Po, z) == ((True, len(z)) if kick < 0.01 else (False, 0))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("lane", [0, 17, 63])
+@pytest.mark.parametrize("slope", [0.0115, 0.013])  # leaves the limits inside the quadrupole, at its entry
+def test_one_irregular_particle_in_a_wavefront(ehlib, lane, slope):
+    rng = np.random.default_rng(lane)
+    rows = np.zeros((192, S.NPROP))  # the first and the last wavefront are regular
+    rows[:, :6] = rng.standard_normal((192, 6)) * [1e-3, 2e-4, 1e-3, 2e-4, 1e-3, 1e-3]
+    rows[64 + lane, :4] = [2e-3, slope, -3e-3, -slope]
+    rows[:, 6] = np.arange(1, 193)
+    lat = Lattice([ELEMENTS[k][0] for k in ("quad", "bend_k1", "sext", "quad_rad")])
+    ref, nref, _, _ = oracle.do_tracking(rows, lat, 2, Po)
+    beam = tracking.Beam(rows)
+    n, _, _ = tracking.track(beam, lat, 2, Po, mode="fused", turns_per_launch=2)
+    got = beam.download()
+    beam.free()
+    assert n == nref == 192
+    check(got, ref, "lane %d slope %g" % (lane, slope))
+
+
 UNBOUNDED = [(np.inf, 0.02), (0.02, np.inf), (np.inf, np.inf), (np.nan, 0.02), (np.finfo(float).max, 0.02)]
 
 
