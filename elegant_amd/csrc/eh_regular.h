@@ -67,10 +67,10 @@
 /* limits of the regular path: 1 + delta; canonical momenta, about the slopes (a
  * bend's QX swings by its sub-step angles on the design orbit already); and the
  * smallest non-zero momentum, whose quotients are far from underflow.  With them
- * |sin phi| < 2^-4 and the series argument below is < 2^-11 (< 2^-7 with WIDE).
- * Comparisons are or-ed into one mask (keeping running maxima and minima instead
- * takes fewer scalar instructions, but v_max_f64 and v_min_f64 cost more than
- * v_cmp: 1e6 particles 4 % slower). */
+ * |sin phi| < 2^-4 and the series argument of eh_reg_root is < 2^-11 (< 2^-8 with
+ * WIDE, where QX takes part), asserted below.  Comparisons are or-ed into one mask
+ * (keeping running maxima and minima instead takes fewer scalar instructions, but
+ * v_max_f64 and v_min_f64 cost more than v_cmp: 1e6 particles 4 % slower). */
 #define EH_REG_B1_MIN 0.875
 #define EH_REG_B1_MAX 1.25
 #define EH_REG_QMAX 0.0117
@@ -83,6 +83,11 @@
 /* what the host leaves for the slopes of a small beam where the design orbit itself
  * comes near a limit */
 #define EH_REG_OWN 1e-3
+static_assert(2 * EH_REG_QMAX * EH_REG_QMAX / (EH_REG_B1_MIN * EH_REG_B1_MIN) < 0x1p-11, "series of eh_reg_root");
+static_assert((EH_REG_QXMAX * EH_REG_QXMAX + EH_REG_QMAX * EH_REG_QMAX) / (EH_REG_B1_MIN * EH_REG_B1_MIN) < 0x1p-8,
+              "series of eh_reg_root<true>");
+/* f >= 0.98 (1 + delta) by the above */
+static_assert(EH_REG_QXMAX / (0.98 * EH_REG_B1_MIN) < EH_REG_ANGLE, "short series of asin");
 /* dense 5 x 5 field block: the terms a gradient alone leaves, (i, j) = (0, 0..4),
  * (1, 0), (1, 2), (1, 3), (2, 2) */
 #define EH_LIVE_GRADIENT 0x9bfu

@@ -378,6 +378,42 @@ extern "C" long bh_regular_arithmetic(long n, unsigned seed) {
   return bad;
 }
 
+/* the same for what radiation adds: the wide root, with QX up to its own limit, and the
+ * reciprocal of 1 + delta after a kick of up to EH_REG_DLOSS, from the exact one and
+ * down a chain of kicks; a larger kick has to be refused */
+extern "C" long bh_regular_radiation(long n, unsigned seed) {
+  std::mt19937_64 rng(seed);
+  auto uni = [&](double lo, double hi) { return lo + (hi - lo) * (double)(rng() >> 11) * 0x1p-53; };
+  auto num = [&]() { return std::ldexp(uni(0.5, 1), -(int)(rng() % 300)) * ((rng() & 1) ? 1 : -1); };
+  long bad = 0;
+  for (long k = 0; k < n; k++) {
+    double b = (k & 7) == 0 ? 1.0 + std::ldexp((double)(int)(rng() % 17) - 8, -53) : uni(EH_REG_B1_MIN, EH_REG_B1_MAX);
+    double rh = 1.0 / b;
+    for (int kick = 0; kick < 4; kick++) {
+      const double b0 = b;
+      b = b * (1 - std::ldexp(uni(0.5, 0.999), -(int)(rng() % 40)) * EH_REG_DLOSS);
+      if ((k & 31) == 1 && kick == 3)
+        b = 1.0 - std::ldexp((double)(rng() % 8), -53); /* far off, or by luck near */
+      const bool near = std::fabs(b / b0 - 1) < 0.9999 * EH_REG_DLOSS, far = std::fabs(b / b0 - 1) > 1.0001 * EH_REG_DLOSS;
+      const bool ok = eh_reg_next_recip(b, rh);
+      bad += (near && !ok) || (far && ok);
+      if (!ok)
+        break;
+      const double a = num();
+      bad += eh_bits(eh_reg_div(a, b, rh)) != eh_bits(a / b);
+      const double qx = ((k & 2) ? 1.0 : std::ldexp(uni(0.5, 1), -(int)(rng() % 60))) * EH_REG_QXMAX;
+      const double qy = ((k & 4) ? 1.0 : std::ldexp(uni(0.5, 1), -(int)(rng() % 60))) * EH_REG_QMAX;
+      const double r = b * b - qx * qx - qy * qy;
+      double f, y;
+      eh_reg_root<true>(r, (qx * qx + qy * qy) * (rh * rh), rh, f, y);
+      bad += eh_bits(f) != eh_bits(std::sqrt(r));
+      const double c = num();
+      bad += eh_bits(eh_reg_div(c, f, y)) != eh_bits(c / f);
+    }
+  }
+  return bad;
+}
+
 /* how many of n particles (rows of 6 coordinates) the regular path takes
  * through one kick multipole or bend (0 if the element has no regular path);
  * taken[i] tells which */

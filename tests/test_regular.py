@@ -106,6 +106,10 @@ def test_quotients_and_roots_are_correctly_rounded():
     assert harness().bh_regular_arithmetic(400000, 5) == 0
 
 
+def test_quotients_and_roots_of_radiating_particles_are_correctly_rounded():
+    assert harness().bh_regular_radiation(200000, 7) == 0
+
+
 @pytest.mark.parametrize("name", sorted(ELEMENTS))
 def test_host_build_matches_oracle(name):
     rows = particles()
