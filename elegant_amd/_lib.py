@@ -26,6 +26,7 @@ EXPORTS = [
     "eh_multipole_tracking", "eh_offset_beam", "eh_rotate_beam", "eh_replay_sequence", "eh_set_central_momentum",
     "eh_track_particles", "eh_beam_row_order", "eh_do_tracking_noalloc", "eh_elimit_amplitudes",
     "eh_get_phase_reference", "eh_set_phase_reference", "eh_delete_phase_references", "eh_do_match_energy",
+    "eh_diag_host_columns",
 ]
 
 
@@ -115,6 +116,8 @@ def load():
     lib.eh_selftest_math.restype = L
     lib.eh_diag_copy.argtypes = [L, C.c_int]
     lib.eh_diag_copy.restype = L
+    lib.eh_diag_host_columns.argtypes = [vp, vp]
+    lib.eh_diag_host_columns.restype = L
     lib.eh_batch_create.argtypes = [L, vp]
     lib.eh_batch_create.restype = vp
     lib.eh_batch_free.argtypes = [vp]

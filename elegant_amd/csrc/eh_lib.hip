@@ -2427,8 +2427,7 @@ extern "C" long eh_elimit_amplitudes(eh_beam *b, double xmax, double ymax, long 
  * (an error if row 0 has the largest); FIRST always fails, as the reference's
  * loop, which never stops early, does (src/simple_rfca.c:101-111) */
 static long reference_order(eh_beam *b, std::vector<int32_t> &slot_at_row, std::vector<int32_t> &alive_row0,
-                            std::vector<int32_t> &dev_index_alive, std::vector<int32_t> *pred = nullptr,
-                            std::vector<int32_t> *order = nullptr);
+                            std::vector<int32_t> &dev_index_alive);
 static long device_order(const eh_rows &w, std::vector<int32_t> &slot_at_row, std::vector<int32_t> &pred,
                          std::vector<int32_t> &order, std::vector<int32_t> &gidx, std::vector<int32_t> &gev);
 static long check_missing(const eh_rows &w, const char *what);
@@ -2873,7 +2872,7 @@ static void replay_order(long N, std::vector<std::pair<int32_t, int32_t>> &lost,
 /* slot_at_row[r] = identity (upload row) of the particle in row r of the
  * reference's arrangement; idx[identity] = index in the alive buffer or -1 */
 static long reference_order(eh_beam *b, std::vector<int32_t> &slot_at_row, std::vector<int32_t> &alive_row0,
-                            std::vector<int32_t> &idx, std::vector<int32_t> *pred, std::vector<int32_t> *order) {
+                            std::vector<int32_t> &idx) {
   long N = b->n_alive + b->n_lost;
   alive_row0.resize(b->n_alive);
   std::vector<int32_t> grow0(b->n_lost), gev(b->n_lost);
@@ -2896,7 +2895,7 @@ static long reference_order(eh_beam *b, std::vector<int32_t> &slot_at_row, std::
       return fail(EH_ERR_STATE, "corrupt particle identity");
     lost[k] = std::make_pair(gev[k], grow0[k]);
   }
-  replay_order(N, lost, slot_at_row, pred, order);
+  replay_order(N, lost, slot_at_row);
   return EH_OK;
 }
 
@@ -4067,6 +4066,20 @@ extern "C" void eh_batch_free(eh_batch *b) {
   if (b->stream)
     (void)hipStreamDestroy(b->stream);
   delete b;
+}
+
+extern "C" long eh_diag_host_columns(eh_beam *beam, eh_batch *batch) {
+  double **cols[2] = {beam ? &beam->d_cols : nullptr, batch ? &batch->d_cols : nullptr};
+  if ((beam && beam->n_alive + beam->n_lost) || (batch && (batch->cur || batch->n_lost)))
+    return fail(EH_ERR_STATE, "eh_diag_host_columns: rows are already on the device");
+  for (double **c : cols)
+    if (c && *c) {
+      HIPCHK(hipFree(*c));
+      *c = nullptr;
+    }
+  if (batch)
+    batch->cols.assign(4 * (size_t)batch->n_total, 0.0);
+  return EH_OK;
 }
 
 extern "C" long eh_batch_upload(eh_batch *b, long v, const double *flat, long n) {

@@ -525,6 +525,11 @@ long eh_selftest_math(const double *x, const double *y, long n, double *out);
  * known HBM traffic for calibrating memory counters (no reference counterpart) */
 long eh_diag_copy(long n, int reps);
 
+/* columns 6 to 9 of the rows kept on the host from the next upload on, as they are
+ * for a beam or batch whose columns do not fit on the device; before any upload
+ * (no reference counterpart, for testing) */
+long eh_diag_host_columns(eh_beam *beam, eh_batch *batch);
+
 #ifdef __cplusplus
 }
 #endif

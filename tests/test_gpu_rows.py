@@ -99,3 +99,45 @@ def test_batch_rows(ehlib, oracle_mod, counts):
         ref, nref, _, _ = oracle_mod.do_tracking(rows[v], ref_lat[v], 2, Po)
         assert_rows_identical(batch.download(v), ref, batch.n_alive(v), nref, "variant %d" % v)
     batch.free()
+
+
+@pytest.mark.parametrize("n", [1, 63, 262145])
+@pytest.mark.parametrize("flat", [True, False])
+def test_columns_on_the_host(ehlib, oracle_mod, n, flat):
+    """a beam whose columns 6 to 9 did not fit on the device: rows consecutive or by
+    pointer, up again after a run"""
+    rows = rows_of(n, 6e-3)
+    place = np.arange(n) if flat else np.random.default_rng(1).permutation(n)
+    store = np.zeros((n, S.NPROP + (0 if flat else 2)))
+    ptr = (store.ctypes.data + place.astype(np.uint64) * np.uint64(store.strides[0])).astype(np.uint64)
+    L = tracking.lib()
+    L.eh_beam_upload.argtypes = [C.c_void_p, C.c_void_p, C.c_long]
+    L.eh_beam_download.argtypes = [C.c_void_p, C.c_void_p, C.c_long]
+    beam = tracking.Beam(np.zeros((0, S.NPROP)), capacity=n + 5)
+    _lib.check(L.eh_diag_host_columns(beam.handle, None))
+    ref, nref, _, _ = oracle_mod.do_tracking(rows, line(), 1, Po)
+    for _ in range(2):
+        store[place, :S.NPROP] = rows
+        _lib.check(L.eh_beam_upload(beam.handle, ptr.ctypes.data, n))
+        na, _, _ = tracking.track(beam, line(), 1, Po)
+        store[:] = -7.0
+        _lib.check(L.eh_beam_download(beam.handle, ptr.ctypes.data, n))
+        assert_rows_identical(store[place, :S.NPROP], ref, na, nref, "n=%d flat=%d" % (n, flat))
+    assert L.eh_diag_host_columns(beam.handle, None) < 0
+    beam.free()
+
+
+def test_batch_columns_on_the_host(ehlib, oracle_mod):
+    counts = [300, 0, 262150, 65]
+    rows = [rows_of(n, (6e-3, 1e-4)[v % 2]) if n else np.zeros((0, S.NPROP)) for v, n in enumerate(counts)]
+    batch = tracking.Batch(rows)
+    L = tracking.lib()
+    _lib.check(L.eh_diag_host_columns(None, batch._h))
+    for v, r in enumerate(rows):
+        r = np.ascontiguousarray(r)
+        _lib.check(L.eh_batch_upload(batch._h, v, r.ctypes.data, len(r)))
+    batch.track([line() for _ in counts], 2, Po)
+    for v in reversed(range(len(counts))):
+        ref, nref, _, _ = oracle_mod.do_tracking(rows[v], line(), 2, Po)
+        assert_rows_identical(batch.download(v), ref, batch.n_alive(v), nref, "variant %d" % v)
+    batch.free()
