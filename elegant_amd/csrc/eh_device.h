@@ -642,7 +642,7 @@ EH_HD void eh_mface2(eh_p6 &p, const eh_desc &d, bool s_too) {
   }
 }
 
-template <bool RAD>
+template <bool RAD, bool FULL>
 EH_HD bool eh_mult_regular_n(const eh_desc &d, int pi, double &x, double &xp, double &y, double &yp, double &s,
                              double &dp);
 
@@ -672,7 +672,7 @@ EH_HD int eh_multipole_t(eh_p6 &p, const eh_desc &d, int pi, const double *__res
   int how = 0; /* 0: coord untouched, 1: x,y written, 2: all written */
   bool regular = false;
   if (d.regular)
-    regular = eh_mult_regular_n<RAD>(d, pi, x, xp, y, yp, s, dp);
+    regular = eh_mult_regular_n<RAD, FULL>(d, pi, x, xp, y, yp, s, dp);
   if (regular) {
     how = 2;
   } else if (eh_isnan(x) || eh_isnan(xp) || eh_isnan(y) || eh_isnan(yp) || eh_fabs(x) > 10.0 || eh_fabs(y) > 10.0 ||
@@ -1417,7 +1417,7 @@ EH_HD bool eh_csbend_t(eh_p6 &p, const eh_desc &d, int pi, const eh_fterm *__res
   double dist = 0, dz_lost = 0;
   bool lost = false, regular = false;
   if (d.regular)
-    regular = eh_csb_regular_n<RAD>(d, pi, terms, X, QX, Y, QY, DP, dist);
+    regular = eh_csb_regular_n<RAD, FULL>(d, pi, terms, X, QX, Y, QY, DP, dist);
   /* integrate_csbend_ordn; the reciprocal pair of 1 + DPoP is for the radiation
    * block's round trip after each kick */
   double rh = 0, rl = 0;

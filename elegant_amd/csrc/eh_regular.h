@@ -45,10 +45,10 @@
  * lost ever does; of slopes of 5 mrad rms nearly every wavefront has one.  Kernel
  * times of short lines of such beams, 2 turns, 4e5 particles: quadrupoles and
  * sextupoles, 5 mrad, 0.58 ms (0.60 with the general integrators alone, 0.70 when
- * the other particles of the wavefront went on here); with bends, 3 mrad, 1.51 (1.51,
- * 1.78); 20 mrad, 1.84 (1.85, 2.45).  1e4 particles, one wavefront alone on its SIMD:
- * 0.19 (0.20, 0.24), 0.52 (0.48, 0.65) and 0.63 (0.61, 0.77).  Looking again at every
- * slice would win back 0.03 of the 0.52 and cost regular beams 1 to 3 %.
+ * the other particles of the wavefront went on here); with bends, 3 mrad, 1.54 (1.51,
+ * 1.79); 20 mrad, 1.88 (1.85, 2.47).  1e4 particles, one wavefront alone on its SIMD:
+ * 0.19 (0.20, 0.24), 0.55 (0.48, 0.65) and 0.66 (0.61, 0.77).  Looking again at every
+ * slice would win back 0.04 of the 0.55 and cost regular beams 1 to 3 %.
  *
  * With SYNCH_RAD the momentum changes at every kick; its reciprocal follows by a
  * Newton step from the last one.  MBA ring with radiation and edges, 5e4
@@ -244,7 +244,13 @@ EH_HD eh_reg_slopes eh_reg_m2s(double qx, double qy, double b1s, double rh, doub
 }
 
 /* Whether any of the wavefront's particles is beyond the limits at entry.  It needs
- * the general integrator, which costs the same for all of them: nobody goes on here. */
+ * the general integrator, which costs the same for all of them: nobody goes on here.
+ * How the compiler lays the code out after it decides a few per cent: told that the
+ * branch is unlikely (bends) or that the mask is clear behind it (multipoles), lean
+ * kernels gain 1 to 2 % with regular beams (FODO study 9.81 -> 9.71 ms, 30401 particles
+ * through the MBA ring 15.25 -> 15.06, batch 30.4 -> 30.0), while the general integrators
+ * of the full ones (FULL) lose 5 to 8 % (elliptical aperture, 1e4 particles 11.1 ->
+ * 12.0); these are told neither. */
 EH_HD bool eh_reg_any(bool bad) {
 #if defined(__HIP_DEVICE_COMPILE__)
   return __ballot(bad) != 0;
@@ -281,7 +287,7 @@ template <int ORDER> EH_HD void eh_reg_mfield(double x, double y, double &Fx, do
  * otherwise.  (1 + x'^2 + y'^2)^1/2 of a sub-step is (1 + delta) / f up to
  * roundings, which one correction step removes.  The exit's slopes are those of
  * the last kick. */
-template <int ORDER, bool RAD>
+template <int ORDER, bool RAD, bool FULL>
 EH_HD bool eh_mult_regular(const eh_desc &d, int pi, double &x_, double &xp_, double &y_, double &yp_, double &s_,
                            double &dp_) {
   double dp = dp_;
@@ -296,6 +302,8 @@ EH_HD bool eh_mult_regular(const eh_desc &d, int pi, double &x_, double &xp_, do
                eh_reg_sized(eh_fabs(yp_)));
   if (eh_reg_any(bad))
     return false;
+  if constexpr (!FULL)
+    bad = false; /* as it is for everyone now */
   double b1s = b1 * b1, rh = 1.0 / b1, rh2 = rh * rh, hrh = 0.5 * rh;
   double qx, qy;
   {
@@ -386,28 +394,28 @@ EH_HD bool eh_mult_regular(const eh_desc &d, int pi, double &x_, double &xp_, do
   return true;
 }
 
-template <bool RAD>
+template <bool RAD, bool FULL>
 EH_HD bool eh_mult_regular_n(const eh_desc &d, int pi, double &x, double &xp, double &y, double &yp, double &s,
                              double &dp) {
   if (d.regular == 1)
-    return eh_mult_regular<1, RAD>(d, pi, x, xp, y, yp, s, dp);
+    return eh_mult_regular<1, RAD, FULL>(d, pi, x, xp, y, yp, s, dp);
   if (d.regular == 2)
-    return eh_mult_regular<2, RAD>(d, pi, x, xp, y, yp, s, dp);
-  return eh_mult_regular<3, RAD>(d, pi, x, xp, y, yp, s, dp);
+    return eh_mult_regular<2, RAD, FULL>(d, pi, x, xp, y, yp, s, dp);
+  return eh_mult_regular<3, RAD, FULL>(d, pi, x, xp, y, yp, s, dp);
 }
 
 /* integrate_csbend_ordn without losses for a regular particle, slopes to momenta
  * before it and back after it: X, xp, Y, yp and the path `dist` advance through
  * the bend if it returns true and are left alone otherwise.  FIELD as
  * eh_desc.regular. */
-template <int FIELD, bool RAD>
+template <int FIELD, bool RAD, bool FULL>
 EH_HD bool eh_csb_regular(const eh_desc &d, int pi, const eh_fterm *__restrict__ terms, double &X_, double &xp_,
                           double &Y_, double &yp_, double &DP_, double &dist_) {
   double X = X_, QX, Y = Y_, QY, DP = DP_, dist = 0;
   double b1 = 1 + DP;
   bool bad = !(b1 >= EH_REG_B1_MIN && b1 <= EH_REG_B1_MAX && eh_fabs(xp_) <= EH_REG_QMAX &&
                eh_fabs(yp_) <= EH_REG_QMAX && eh_reg_sized(eh_fabs(yp_)));
-  if (eh_reg_any(bad))
+  if (FULL ? eh_reg_any(bad) : __builtin_expect(eh_reg_any(bad), 0))
     return false;
   const double rho0 = d.rho0, rho_a = d.rho_actual, r0h = d.rho0_rh, rah = d.rhoa_rh;
   const double apx = d.reg_apx[pi], apy = d.reg_apy[pi];
@@ -523,14 +531,14 @@ EH_HD bool eh_csb_regular(const eh_desc &d, int pi, const eh_fterm *__restrict__
   return true;
 }
 
-template <bool RAD>
+template <bool RAD, bool FULL>
 EH_HD bool eh_csb_regular_n(const eh_desc &d, int pi, const eh_fterm *__restrict__ terms, double &X, double &xp,
                             double &Y, double &yp, double &DP, double &dist) {
   if (d.regular == 2)
-    return eh_csb_regular<2, RAD>(d, pi, terms, X, xp, Y, yp, DP, dist);
+    return eh_csb_regular<2, RAD, FULL>(d, pi, terms, X, xp, Y, yp, DP, dist);
   if (d.regular == 1)
-    return eh_csb_regular<1, RAD>(d, pi, terms, X, xp, Y, yp, DP, dist);
-  return eh_csb_regular<3, RAD>(d, pi, terms, X, xp, Y, yp, DP, dist);
+    return eh_csb_regular<1, RAD, FULL>(d, pi, terms, X, xp, Y, yp, DP, dist);
+  return eh_csb_regular<3, RAD, FULL>(d, pi, terms, X, xp, Y, yp, DP, dist);
 }
 
 #endif
