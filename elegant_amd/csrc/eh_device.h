@@ -59,9 +59,10 @@ typedef struct {
    * the regular path, in the order it is read, so that an element costs a few
    * neighbouring lines of the scalar cache (16 KB for two CUs: the heads of a
    * ring's distinct elements stay there from cell to cell).  With these fields
-   * spread over the descriptor, one wavefront alone on its SIMD spent 2900 cycles
-   * on a drift (1.2 us), nearly all of them waiting for one scalar load after
-   * another; it is 0.76 us now, and 1e6 particles take 3.8 us instead of 5.9. */
+   * spread over the descriptor, one wavefront alone on its SIMD spends 2900 cycles
+   * on a drift, nearly all of them waiting for one scalar load after another;
+   * gathered here they save it a third (1.2 -> 0.76 us), and 1e6 particles as much.
+   * What a drift takes in all is with drift_step. */
   int32_t type; /* eh_type */
   int32_t counted; /* counts as a particle-element unit (not MARK/MAXAMP) */
   /* how the regular path runs this element (eh_regular.h): 0 not at all; bends
@@ -642,7 +643,7 @@ EH_HD void eh_mface2(eh_p6 &p, const eh_desc &d, bool s_too) {
   }
 }
 
-template <bool RAD, bool FULL>
+template <bool RAD>
 EH_HD bool eh_mult_regular_n(const eh_desc &d, int pi, double &x, double &xp, double &y, double &yp, double &s,
                              double &dp);
 
@@ -672,7 +673,7 @@ EH_HD int eh_multipole_t(eh_p6 &p, const eh_desc &d, int pi, const double *__res
   int how = 0; /* 0: coord untouched, 1: x,y written, 2: all written */
   bool regular = false;
   if (d.regular)
-    regular = eh_mult_regular_n<RAD, FULL>(d, pi, x, xp, y, yp, s, dp);
+    regular = eh_mult_regular_n<RAD>(d, pi, x, xp, y, yp, s, dp);
   if (regular) {
     how = 2;
   } else if (eh_isnan(x) || eh_isnan(xp) || eh_isnan(y) || eh_isnan(yp) || eh_fabs(x) > 10.0 || eh_fabs(y) > 10.0 ||

@@ -32,12 +32,13 @@
  * What bounds these loops is the number of instructions: a dependent FP64 fma
  * issues every 5 cycles from one wavefront and every 4 from several, so that a
  * launch of few particles gains nothing from independent operations and one of
- * many nothing from latency hiding.  A sub-step of a gradient bend takes 165
- * vector and 30 scalar instructions here against 270 and 215 in the general
- * integrator, whose branches also keep the compiler from holding the polynomial
- * constants in scalar registers.  Measured (MI355X, MBA ring, fused, 2 turns): 1e6
- * particles 283 -> 166 ms, 30 401 particles (one wavefront on half of the SIMDs)
- * 48.4 -> 21.4 ms; FODO ring, 1e4 particles, 40 turns 27.2 -> 13.4 ms.
+ * many nothing from latency hiding.  A sub-step of a gradient bend takes 144
+ * instructions here, 120 of them FP64, against 270 vector and 215 scalar ones in the
+ * general integrator, whose branches also keep the compiler from holding the
+ * polynomial constants in scalar registers.  Kernel times with the general
+ * integrators alone and now (MI355X, MBA ring, fused, 2 turns): 1e6 particles 283 and
+ * 137 ms, 30 401 particles (one wavefront on half of the SIMDs) 48.4 and 15.1 ms; FODO
+ * ring, 1e4 particles, 40 turns 27.2 and 9.7 ms.
  *
  * A wavefront runs the general integrator as soon as one of its particles is beyond
  * the limits at an element's entry, and both integrators where one leaves them
@@ -52,7 +53,7 @@
  *
  * With SYNCH_RAD the momentum changes at every kick; its reciprocal follows by a
  * Newton step from the last one.  MBA ring with radiation and edges, 5e4
- * particles, one turn: 27.1 -> 14.6 ms.
+ * particles, one turn: 27.1 and 11.2 ms.
  *
  * The starting values need no hardware estimate (v_rcp_f64 and v_rsq_f64 give 24
  * bits and take the issue time of four fma): a bend's and a multipole's root is
@@ -245,12 +246,13 @@ EH_HD eh_reg_slopes eh_reg_m2s(double qx, double qy, double b1s, double rh, doub
 
 /* Whether any of the wavefront's particles is beyond the limits at entry.  It needs
  * the general integrator, which costs the same for all of them: nobody goes on here.
- * How the compiler lays the code out after it decides a few per cent: told that the
- * branch is unlikely (bends) or that the mask is clear behind it (multipoles), lean
+ * How the compiler lays the code out after it decides a few per cent.  Told that the
+ * mask is clear behind the vote (multipoles) and that the exit is unlikely (bends) lean
  * kernels gain 1 to 2 % with regular beams (FODO study 9.81 -> 9.71 ms, 30401 particles
- * through the MBA ring 15.25 -> 15.06, batch 30.4 -> 30.0), while the general integrators
- * of the full ones (FULL) lose 5 to 8 % (elliptical aperture, 1e4 particles 11.1 ->
- * 12.0); these are told neither. */
+ * through the MBA ring 15.25 -> 15.06, batch 30.4 -> 30.0).  In full kernels (FULL) an
+ * unlikely exit costs the general integrators 5 to 8 % (elliptical aperture, 1e4
+ * particles 11.1 -> 12.0), and a clear mask in the bends, too, gains 1 to 3 % (radiating
+ * MBA ring 11.24 -> 11.13). */
 EH_HD bool eh_reg_any(bool bad) {
 #if defined(__HIP_DEVICE_COMPILE__)
   return __ballot(bad) != 0;
@@ -287,7 +289,7 @@ template <int ORDER> EH_HD void eh_reg_mfield(double x, double y, double &Fx, do
  * otherwise.  (1 + x'^2 + y'^2)^1/2 of a sub-step is (1 + delta) / f up to
  * roundings, which one correction step removes.  The exit's slopes are those of
  * the last kick. */
-template <int ORDER, bool RAD, bool FULL>
+template <int ORDER, bool RAD>
 EH_HD bool eh_mult_regular(const eh_desc &d, int pi, double &x_, double &xp_, double &y_, double &yp_, double &s_,
                            double &dp_) {
   double dp = dp_;
@@ -302,8 +304,7 @@ EH_HD bool eh_mult_regular(const eh_desc &d, int pi, double &x_, double &xp_, do
                eh_reg_sized(eh_fabs(yp_)));
   if (eh_reg_any(bad))
     return false;
-  if constexpr (!FULL)
-    bad = false; /* as it is for everyone now */
+  bad = false; /* as it is for everyone now */
   double b1s = b1 * b1, rh = 1.0 / b1, rh2 = rh * rh, hrh = 0.5 * rh;
   double qx, qy;
   {
@@ -394,14 +395,14 @@ EH_HD bool eh_mult_regular(const eh_desc &d, int pi, double &x_, double &xp_, do
   return true;
 }
 
-template <bool RAD, bool FULL>
+template <bool RAD>
 EH_HD bool eh_mult_regular_n(const eh_desc &d, int pi, double &x, double &xp, double &y, double &yp, double &s,
                              double &dp) {
   if (d.regular == 1)
-    return eh_mult_regular<1, RAD, FULL>(d, pi, x, xp, y, yp, s, dp);
+    return eh_mult_regular<1, RAD>(d, pi, x, xp, y, yp, s, dp);
   if (d.regular == 2)
-    return eh_mult_regular<2, RAD, FULL>(d, pi, x, xp, y, yp, s, dp);
-  return eh_mult_regular<3, RAD, FULL>(d, pi, x, xp, y, yp, s, dp);
+    return eh_mult_regular<2, RAD>(d, pi, x, xp, y, yp, s, dp);
+  return eh_mult_regular<3, RAD>(d, pi, x, xp, y, yp, s, dp);
 }
 
 /* integrate_csbend_ordn without losses for a regular particle, slopes to momenta
@@ -417,6 +418,8 @@ EH_HD bool eh_csb_regular(const eh_desc &d, int pi, const eh_fterm *__restrict__
                eh_fabs(yp_) <= EH_REG_QMAX && eh_reg_sized(eh_fabs(yp_)));
   if (FULL ? eh_reg_any(bad) : __builtin_expect(eh_reg_any(bad), 0))
     return false;
+  if constexpr (FULL)
+    bad = false;
   const double rho0 = d.rho0, rho_a = d.rho_actual, r0h = d.rho0_rh, rah = d.rhoa_rh;
   const double apx = d.reg_apx[pi], apy = d.reg_apy[pi];
   const double h0 = d.reg_h[0], h1 = d.reg_h[1], k0 = d.reg_k[0], k1 = d.reg_k[1];

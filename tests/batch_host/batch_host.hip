@@ -439,8 +439,8 @@ extern "C" long bh_regular_taken(const double *z, long n, const EH_ELEMENT_LIST 
       taken[i] = d.rad ? eh_csb_regular_n<true, true>(d, 0, terms.data(), x, xp, y, yp, dp, s)
                        : eh_csb_regular_n<false, true>(d, 0, terms.data(), x, xp, y, yp, dp, s);
     } else if (d.regular) {
-      taken[i] = d.rad ? eh_mult_regular_n<true, true>(d, 0, x, xp, y, yp, s, dp)
-                       : eh_mult_regular_n<false, true>(d, 0, x, xp, y, yp, s, dp);
+      taken[i] = d.rad ? eh_mult_regular_n<true>(d, 0, x, xp, y, yp, s, dp)
+                       : eh_mult_regular_n<false>(d, 0, x, xp, y, yp, s, dp);
     }
     count += taken[i];
   }
