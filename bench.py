@@ -15,10 +15,10 @@ Further legs in the same JSON line:
            (4.9e6 in total), 6D Gaussian beams, all variants in one persistent
            launch per span captured in a HIP graph, launch shape from the
            autotuner;
-  plain    the per-element drop-in path (one kernel per reference call, host
-           synchronisation and compaction after each) on the 10-cell FODO ring
-           with 1e4 particles: the launch-bound small-lattice case the batched
-           path is compared with;
+  plain    element by element (one launch per element with its sweeps, one host
+           visit and compaction per turn) on the 10-cell FODO ring with 1e4
+           particles: the launch-bound small-lattice case the batched path is
+           compared with;
   cpu_baseline  the checker compiled like the reference (gcc -O3 -m64, C-library
            transcendentals) on a bounded strided sample of the headline
            workload, one single-threaded worker per host core.
@@ -240,7 +240,7 @@ def leg_plain(args):
     log("plain timed: %d turns, %d alive, %.3f s wall, %d launches" % (args.plain_steps, n, wall, st["launches"]))
     return {"value": units / wall, "unit": UNIT, "turns": args.plain_steps, "particles": len(rows),
             "survivors": n, "wall_s": round(wall, 4), "launches": st["launches"],
-            "workload": desc + ", per-element drop-in path"}
+            "workload": desc + ", one launch per element"}
 
 
 def leg_adjoint(args):
@@ -463,7 +463,7 @@ def main():
                 "hw_fp64": hw,
                 "pipe": "FP64 VALU, no MFMA (compute-bound: the vector FP64 pipe; peak is MI355X's FP64 "
                         "vector peak)",
-                "kernel": "k_fused" if args.mode == "fused" else "k_plain",
+                "kernel": "k_fused" if args.mode == "fused" else "k_step",
                 "algorithmic_flops_per_unit": round(alg_per_unit, 2),
                 "units_per_launch": round(st["main_units"] / launches),
                 "launches": st["main_launches"],

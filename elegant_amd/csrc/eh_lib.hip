@@ -1461,11 +1461,15 @@ extern "C" long eh_beam_upload(eh_beam *b, double **coord, long n_part) {
 #define EH_BLOCK 256
 /* Occupancy target for the tracking kernels: five wavefronts per SIMD, 96 VGPRs.
  * The regular integrators are bound by instruction issue, which four or five
- * wavefronts fill; a sixth only costs spills around them.  Kernel time in ms at 3,
- * 4, 5 and 6 wavefronts: MBA ring, 2 turns, 1e6 particles 143.7, 139.4, 137.3, 139.5;
- * 30401 particles (one wavefront per SIMD or none) 15.6, 16.0, 15.7, 17.2; with
- * radiation, 5e4 particles, 1 turn 11.0, 11.1, 11.2, 11.7; FODO ring, 1e4 particles,
- * 40 turns 10.1, 10.0, 10.0, 11.9. */
+ * wavefronts fill; a sixth only costs spills.  The general integrators do not need it
+ * either.  Kernel time in ms at 4, 5 and 6 wavefronts.  Regular: MBA ring, 2 turns,
+ * 1e6 particles 139.4, 137.3, 139.5; 30401 particles (one wavefront per SIMD or none)
+ * 15.6, 15.3, 17.2; with radiation, 5e4 particles, 1 turn 11.1, 11.2, 11.7; FODO ring,
+ * 1e4 particles, 40 turns 10.3, 9.8, 11.9.  General, 8 cells of the MBA ring, 2 turns,
+ * 4e5 particles and 1e4: all magnets tilted 28.3, 27.6, 28.8 and 9.1, 9.1, 10.1;
+ * elliptical aperture 32.3, 31.5, 33.3 and 10.9, 11.1, 12.4; tilted and radiating 35.3,
+ * 35.1, 36.9 and 10.4, 10.7, 12.1; order 6, radiating 74.0, 72.8, 75.2 and 21.7, 22.0,
+ * 24.6. */
 #define EH_TRACK_WAVES __attribute__((amdgpu_waves_per_eu(5)))
 
 __device__ __forceinline__ eh_p6 load_p(const eh_soa a, long i) {
@@ -1651,12 +1655,11 @@ __global__ void __launch_bounds__(EH_BLOCK) k_compact(eh_soa a, long n, eh_soa b
 
 /* a DRIF and its sweeps: half of a ring's positions, a dozen operations each.  On
  * its own, ahead of the switch, it works on the coordinates in place; inside, it
- * pays for the copies the compiler makes around the switch.  6400 particles through
- * a drift 0.57 us before, 0.39 now, 1e6 3.3 and 2.2; MBA ring, 2 turns: 30401
- * particles 15.6 -> 15.3 ms, 1e6 137.7 -> 136.1; FODO ring, 1e4 particles, 40 turns
- * 10.0 -> 9.7; forward pass of the adjoint 16.3 -> 15.9.  k_batch, whose wavefronts
- * learn the type from the descriptor, does not gain (29.7 and 30.0) and goes through
- * the switch.  Returns the stage that lost the particle, or -1. */
+ * pays for the copies the compiler makes around the switch.  6400 particles, a
+ * wavefront alone on its SIMD, take 0.40 us through a drift (0.57 inside the switch),
+ * 1e6 take 2.2 (3.3); the rings gain 1 to 3 %.  k_batch, whose wavefronts learn the
+ * type from the descriptor, gains nothing (30.0 ms here, 29.7 in the switch) and goes
+ * through the switch.  Returns the stage that lost the particle, or -1. */
 template <bool RAD>
 __device__ __forceinline__ int drift_step(eh_p6 &p, bool alive, const eh_desc &d, int pass,
                                           const double *__restrict__ zp) {
@@ -1680,9 +1683,9 @@ __device__ __forceinline__ int drift_step(eh_p6 &p, bool alive, const eh_desc &d
  * element's type are therefore read 64 positions at a time, one to a lane, and
  * handed over by a lane read, so that the switch and the element's loads wait for
  * no other load (an offset prefetched as a scalar was spilled as soon as it
- * arrived, which waits for it).  6400 particles through a drift: 0.75 us before,
- * 0.57 now; 30401 through the MBA ring, 8 turns: 16.8 ms before, 15.7 now; 1e6, 2
- * turns, where five wavefronts hide one another's waits: 142 and 139.  `units` (wavefront-
+ * arrived, which waits for it).  That is a quarter of a drift's time for 6400
+ * particles, 7 % of the MBA ring for 30401 (16.8 -> 15.7 ms when it came) and 2 % for
+ * 1e6, where five wavefronts hide one another's waits.  `units` (wavefront-
  * uniform) counts the wavefront's particle-element units; a lost lane keeps
  * where and how in one word (eh_loss_code, decoded by eh_loss_words): a single
  * loop-carried register. */
