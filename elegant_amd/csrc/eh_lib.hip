@@ -3962,14 +3962,16 @@ static void keep_lines(eh_kept_lines &k, EH_ELEMENT_LIST *const *bl, long nvar, 
   k.nvar = nvar;
   k.ne = ne;
   k.bytes.clear();
-  auto put = [&](const void *p, size_t n) { k.bytes.insert(k.bytes.end(), (const char *)p, (const char *)p + n); };
+  k.bytes.reserve((size_t)nvar * ne * 64); /* pages are taken as they fill; growing would copy them */
   for (long v = 0; v < nvar; v++)
     for (long e = 0; e < ne; e++) {
-      const char how = kept_as(bl, v, e);
-      put(&how, 1);
-      put(&bl[v][e].type, sizeof(int32_t));
-      if (how == EH_KEPT_OWN)
-        put(bl[v][e].p_elem, elem_struct_size(bl[v][e].type));
+      char head[1 + sizeof(int32_t)] = {kept_as(bl, v, e)};
+      std::memcpy(head + 1, &bl[v][e].type, sizeof(int32_t));
+      k.bytes.insert(k.bytes.end(), head, head + sizeof head);
+      if (head[0] == EH_KEPT_OWN) {
+        const char *p = (const char *)bl[v][e].p_elem;
+        k.bytes.insert(k.bytes.end(), p, p + elem_struct_size(bl[v][e].type));
+      }
     }
 }
 
